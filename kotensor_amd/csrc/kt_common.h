@@ -61,6 +61,11 @@ struct WaitLimits {
 };
 WaitLimits wait_limits();
 
+// Whether the stream's workspace can hold `bytes` of general area now (while it is being
+// captured it cannot grow; a caller's fixed workspace never does), for calls that have a
+// way to do without.
+bool workspace_fits(hipStream_t stream, size_t bytes);
+
 // Validated view of a kt_qweight, with the derived layout numbers.
 struct WeightView {
     const uint8_t* q;
@@ -125,6 +130,10 @@ int32_t launch_generic(const float* a, int32_t m, const WeightView& w, float* c,
                        float alpha, const float* bias, hipStream_t st);
 int32_t launch_transposed(const float* dy, int32_t m, const WeightView& w, float* dx,
                           int32_t accumulate, hipStream_t st);
+// The transposed product in fp32 precision on the bf16 matrix units (kt_split.hip).
+bool transposed_split_preferred(int32_t m, const WeightView& w);
+int32_t launch_transposed_split(const float* dy, int32_t m, const WeightView& w, float* dx, int32_t accumulate,
+                                hipStream_t st);
 int32_t launch_dequantize_rows(const WeightView& w, const int32_t* rows, int32_t count, float* out,
                                hipStream_t st);
 int32_t launch_dequantize_columns(const WeightView& w, const int32_t* cols, int32_t count, float* out,

@@ -59,7 +59,8 @@ __device__ __forceinline__ float row_value(const uint8_t* q, const float* s, con
 }
 
 // One workgroup per (weight row l, chunk of 8 dy rows): partial dots over n, then
-// a fixed-order tree in LDS.
+// a fixed-order tree in LDS. For small work and group sizes that are not whole 32-row
+// blocks; kt_split.hip has the larger products.
 constexpr int TR_ROWS = 8;
 __global__ void __launch_bounds__(256)
     transposed_kernel(const float* __restrict__ dy, int32_t M, const uint8_t* __restrict__ q, const float* __restrict__ s,
@@ -148,6 +149,7 @@ int32_t launch_generic(const float* a, int32_t m, const WeightView& w, float* c,
 
 int32_t launch_transposed(const float* dy, int32_t m, const WeightView& w, float* dx, int32_t accumulate,
                           hipStream_t st) {
+    if (transposed_split_preferred(m, w)) return launch_transposed_split(dy, m, w, dx, accumulate, st);
     dim3 grid;
     int32_t status = grid_1d(static_cast<int64_t>(w.K) * ceil_div(m, TR_ROWS), &grid);
     if (status) return status;

@@ -135,6 +135,17 @@ int32_t workspace(hipStream_t stream, size_t bytes, void** out) {
     return KT_OK;
 }
 
+bool workspace_fits(hipStream_t stream, size_t bytes) {
+    if (t_fixed) return bytes <= t_fixed->bytes - COUNTER_BYTES - t_fixed->zero_bytes;
+    int device = 0;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipGetDevice(&device) != hipSuccess || hipStreamIsCapturing(stream, &capture) != hipSuccess) return false;
+    if (capture == hipStreamCaptureStatusNone) return true;
+    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    const auto it = g_ws.find(std::make_pair(device, stream));
+    return it != g_ws.end() && it->second.ptr && COUNTER_BYTES + it->second.zbytes + bytes <= it->second.bytes;
+}
+
 int32_t workspace_counters(hipStream_t stream, size_t bytes, size_t count, void** general, uint32_t** counters) {
     if (count > MAX_COUNTERS) return fail(KT_ERR_SHAPE, "too many reduction counters");
     if (t_fixed) {

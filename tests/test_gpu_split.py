@@ -1,0 +1,117 @@
+"""The products on the bf16 matrix units (kt_split.hip) against the same sums in 64 bits.
+
+Bound: weights are exact and every other operand is an fp32 number split exactly, so what
+remains are fp32 roundings: one per product and one per addition on a sum's path, at most
+a few dozen of 2^-24 each at these sizes; normwise they add as a random walk, held to 1e-6.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+from conftest import normwise_rel
+from gpu_helpers import banner, same_bits, upload_quantized
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-6
+
+
+def _weights(oracle_lib, k, n, bits, g, seed):
+    rng = np.random.default_rng(seed)
+    w = (rng.standard_normal((k, n), dtype=np.float32) * np.float32(0.02)).astype(np.float32)
+    st, q = oracle_lib.quantize(w, bits, g)
+    assert st == 0
+    return q
+
+
+def _transposed(kt, dy, qt, dx0=None):
+    m, k = dy.shape[0], qt.rows
+    a = kt.DeviceBuffer.from_numpy(dy)
+    dx = kt.DeviceBuffer.from_numpy(np.full((m, k), np.nan, np.float32) if dx0 is None else dx0)
+    kt.MatMul.multiply_by_quantized_transposed(a, qt, dx, m, accumulate=dx0 is not None)
+    kt.synchronize()
+    return dx.download(np.float32).reshape(m, k)
+
+
+# (m, k, n, bits, g): row tiles of 32, 64 and 128, the 128 and 512 weight rows of a tile,
+# steps of 64 columns with every kind of end (odd, one column past a step, fewer than a
+# step), groups of one to four 32-row blocks and of 96, runs of a slice
+TRANSPOSED = [
+    (1, 2300, 4100, 4, 64), (32, 513, 12001, 8, 32), (33, 1000, 2999, 4, 64), (65, 1024, 1025, 8, 64),
+    (128, 385, 4096, 4, 128), (129, 2048, 577, 4, 96), (200, 640, 100, 4, 32), (300, 900, 9, 4, 64),
+    (130, 9000, 64, 8, 128), (257, 512, 4672, 8, 256), (96, 4096, 7001, 4, 32),
+]
+
+
+@pytest.mark.parametrize("m,k,n,bits,g", TRANSPOSED)
+def test_transposed_against_64_bits(kt, oracle_lib, m, k, n, bits, g):
+    banner("split-transposed", m, k, n, bits, g)
+    q = _weights(oracle_lib, k, n, bits, g, m + k + n)
+    qt = upload_quantized(kt, q)
+    rng = np.random.default_rng(m)
+    dy = (rng.standard_normal((m, n)) * np.exp(4 * rng.standard_normal((m, 1)))).astype(np.float32)
+    want = dy.astype(np.float64) @ q.dequantize().astype(np.float64).T
+    got = _transposed(kt, dy, qt)
+    # every row by itself: rows differ in size by orders of magnitude
+    err = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+    print(f"  largest row error {err.max():.2e}", flush=True)
+    assert err.max() <= TOL
+    dx0 = rng.standard_normal((m, k)).astype(np.float32)
+    assert normwise_rel(_transposed(kt, dy, qt, dx0), want + dx0) <= TOL
+    assert same_bits(got, _transposed(kt, dy, qt))
+
+
+def test_transposed_infinities_and_nans(kt, oracle_lib):
+    """An infinite or NaN dY element reaches its row alone, with the products' signs; finite
+    elements next to it, also the largest fp32 numbers, stay exact."""
+    m, k, n = 70, 700, 2001
+    banner("split-transposed-inf")
+    q = _weights(oracle_lib, k, n, 4, 64, 5)
+    qt = upload_quantized(kt, q)
+    dy = np.random.default_rng(6).standard_normal((m, n)).astype(np.float32)
+    plain = _transposed(kt, dy, qt)
+    w = q.dequantize()
+    odd = dy.copy()
+    odd[3, 17], odd[40, 2000], odd[41, 1000] = np.inf, -np.inf, np.nan
+    odd[50] = 0.0
+    odd[50, 1024] = 3.4e38
+    got = _transposed(kt, odd, qt)
+    with np.errstate(invalid="ignore"):
+        assert np.array_equal(got[3], np.float32(np.inf) * w[:, 17], equal_nan=True)
+        assert np.array_equal(got[40], np.float32(-np.inf) * w[:, 2000], equal_nan=True)
+    assert np.isnan(got[41]).all()
+    np.testing.assert_allclose(got[50], np.float32(3.4e38) * w[:, 1024], rtol=3e-7)
+    rest = np.setdiff1d(np.arange(m), [3, 40, 41, 50])
+    assert same_bits(got[rest], plain[rest])
+
+
+def test_transposed_recorded_without_workspace(kt, oracle_lib):
+    """Recorded on a stream that never ran eagerly (no workspace to split into): replays
+    equal the 64-bit result, with eager calls in between."""
+    from kotensor_amd import _lib
+    m, k, n = 64, 1024, 2000
+    q = _weights(oracle_lib, k, n, 4, 64, 9)
+    qt = upload_quantized(kt, q)
+    dy = np.random.default_rng(10).standard_normal((m, n)).astype(np.float32)
+    want = dy.astype(np.float64) @ q.dequantize().astype(np.float64).T
+    a, dx = kt.DeviceBuffer.from_numpy(dy), kt.DeviceBuffer(m * k * 4)
+    stream, graph = kt.Stream.create(), ctypes.c_void_p()
+    kt.synchronize()
+    banner("split-transposed-record")
+    _lib.call("kt_graph_begin", stream.handle)
+    try:
+        kt.MatMul.multiply_by_quantized_transposed(a, qt, dx, m, accumulate=False, stream=stream)
+    finally:
+        _lib.call("kt_graph_end", stream.handle, ctypes.byref(graph))
+    try:
+        for _ in range(3):
+            dx.fill_zero()
+            kt.synchronize()
+            _lib.call("kt_graph_launch", graph, stream.handle)
+            stream.synchronize()
+            assert normwise_rel(dx.download(np.float32).reshape(m, k), want) <= TOL
+            assert normwise_rel(_transposed(kt, dy, qt), want) <= TOL
+    finally:
+        stream.synchronize()
+        _lib.call("kt_graph_destroy", graph)
+        stream.destroy()
