@@ -1,0 +1,33 @@
+"""The fused cross-entropy's passes of many chunks (kt_loss.hip) against the oracle, where a
+pass ends: more rows than 2^25 logits hold, a last chunk of at most 16 rows (its product on
+its own), chunks of at most 16 rows, rows beyond the registers' 32768 logits, a single class.
+
+Bound: as tests/test_gpu_loss.py, the products' 2e-3 normwise."""
+import numpy as np
+import pytest
+
+import oracle
+from conftest import normwise_rel
+from gpu_helpers import banner, same_bits
+from test_gpu_loss import TOL, _run, _setup
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("k,n,rows,bits,g", [
+    (64, 151936, 230, 4, 64),  # 27 rows a chunk, 216 a pass; the second pass has 14
+    (32, 300000, 30, 8, 32),   # 13 rows a chunk
+    (64, 32768, 145, 4, 32),   # 128 rows a chunk and 17 more in one product
+    (64, 32769, 135, 8, 64),   # 127 rows a chunk, 8 more on their own; one logit past the registers
+    (64, 1, 20, 8, 64),
+])
+def test_passes_match_the_oracle(kt, oracle_lib, k, n, rows, bits, g):
+    banner("fused-ce-passes", k, n, rows, bits, g)
+    q, head, bias, hidden, targets = _setup(kt, oracle_lib, k, n, rows, bits, g, k + n)
+    loss, hg, bg = _run(kt, head, hidden, targets)
+    want_loss, want_hg, want_bg = oracle.fused_cross_entropy(hidden, q, targets, bias, threads=16)
+    assert abs(loss - want_loss) <= TOL * max(1.0, abs(want_loss))
+    assert normwise_rel(hg, want_hg) <= TOL
+    assert normwise_rel(bg, want_bg) <= TOL
+    loss2, hg2, bg2 = _run(kt, head, hidden, targets)
+    assert loss2 == loss and same_bits(hg, hg2) and same_bits(bg, bg2)
