@@ -130,7 +130,11 @@ int32_t launch_generic(const float* a, int32_t m, const WeightView& w, float* c,
                        float alpha, const float* bias, hipStream_t st);
 int32_t launch_transposed(const float* dy, int32_t m, const WeightView& w, float* dx,
                           int32_t accumulate, hipStream_t st);
-// The transposed product in fp32 precision on the bf16 matrix units (kt_split.hip).
+// Products in fp32 precision on the bf16 matrix units (kt_split.hip): the transposed one and
+// the forward one of any shape and alignment.
+bool forward_split_preferred(int32_t m, const WeightView& w);
+int32_t launch_forward_split(const float* a, int32_t m, const WeightView& w, float* c, int32_t accumulate, float alpha,
+                             const float* bias, hipStream_t st);
 bool transposed_split_preferred(int32_t m, const WeightView& w);
 int32_t launch_transposed_split(const float* dy, int32_t m, const WeightView& w, float* dx, int32_t accumulate,
                                 hipStream_t st);

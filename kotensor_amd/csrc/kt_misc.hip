@@ -1,9 +1,9 @@
 // kt_misc.hip -- the kernels that complete the API around the fast paths:
-//   * generic_matmul: any shape and alignment (odd widths, group sizes that are
-//     not a multiple of 4, misaligned pointers), one thread per output element,
+//   * generic_matmul: any shape and alignment that kt_split.hip does not take (group sizes
+//     that are not whole 32 rows, fewer than 8 columns), one thread per output element,
 //     group by group with the reference's combine
 //     out += scale * (sum_k a*q - zero * sum_k a)  (MatMul.kt:804-828,942-952);
-//   * transposed: dx = dy . deq(W)^T (MatMul.kt:954-981), 8-bit rows dequantized
+//   * transposed: dx = dy . deq(W)^T (MatMul.kt:954-981) of small work, 8-bit rows dequantized
 //     without zero points as QuantizedTensor.dequantizeRow does (QuantizedTensor.kt:198-202);
 //   * dequantize_rows / dequantize_columns: the embedding gathers
 //     (QuantizedTensor.kt:188-241, Embedding.kt:73-136).
@@ -139,6 +139,7 @@ int32_t grid_1d(int64_t blocks, dim3* grid) {
 
 int32_t launch_generic(const float* a, int32_t m, const WeightView& w, float* c, int32_t accumulate, float alpha,
                        const float* bias, hipStream_t st) {
+    if (forward_split_preferred(m, w)) return launch_forward_split(a, m, w, c, accumulate, alpha, bias, st);
     dim3 grid;
     int32_t status = grid_1d(static_cast<int64_t>(m) * ceil_div(w.N, 256), &grid);
     if (status) return status;

@@ -7,8 +7,11 @@
 // are exact and whose sums are fp32: the precision of an fp32 multiply-add chain at a
 // third of the bf16 rate (about 5 times the fp32 matrix rate).
 //
+//   forward: c[M x N] = a[M x K] . deq(W) (MatMul.multiplyQuantized, Engine/kotensor/src/main/
+//   kotlin/MatMul.kt:479-485) of the shapes and alignments the fp16 GEMM does not take; the
+//   scale of a k-group multiplies the group's sum.
 //   transposed: dX[M x K] = dY[M x N] . deq(W)^T (MatMul.multiplyByQuantizedTransposed,
-//   Engine/kotensor/src/main/kotlin/MatMul.kt:954-981). The sum runs over n, along which
+//   MatMul.kt:954-981). The sum runs over n, along which
 //   the scale changes, so a lane multiplies its dY values by the scales of the k-group
 //   first (one fp32 rounding, in the place of the one of deq(W)) and splits the product.
 #include <algorithm>
@@ -419,10 +422,278 @@ __global__ void __launch_bounds__(THREADS, 2) transposed_split_kernel(SplitArgs 
     }
 }
 
-// out = (accumulate ? out : 0) + the slices' sums, in a fixed order.
+// ---- forward: c[M x N] = (accumulate ? c : 0) + alpha a[M x K] . deq(W) (+ bias) ------------
+struct ForwardArgs {
+    const float* a;
+    const uint8_t* q;
+    const float* s;
+    const int8_t* z;
+    float* c;         // or the slices' sums [splits][M][N]
+    const float* bias;
+    int32_t M, K, N, bpr, g, G, tiles_m, splits, steps, steps_per_split, accumulate;
+    float alpha;
+};
+
+// Workgroup (tile of 32 WM rows of a and 128 WN columns, slice of k): each wave owns 32
+// rows x 128 columns; for INT4 64 bytes of a weight row: 64 low-nibble columns and the 64
+// high-nibble columns of the same bytes. A step is 64 k. The weights come to LDS transposed
+// ([column][k], so that a lane's operand is 16 contiguous bytes): a thread takes 4 (INT4:
+// 2) byte columns of 8 rows, and byte j of lane cq's columns goes to LDS row 32 j + cq, so
+// that 32 lanes write 32 consecutive rows (no bank conflicts) and a lane ends with the sums
+// of adjacent columns. The scale is constant along a group's k, so the group's sum is
+// scaled, with one fp32 multiply-add: SC steps of 16 k share a scale (4 or 2).
+// Bound by the steps' conversions and splits (vector ALU, 350 instructions a wave and step)
+// beside 48 matrix products, at few rows by the conversions and the slices' sum:
+// M = 512, 2048 -> 8191, INT4 g = 64 80 us, 214 TFLOP/s (generic_matmul 2784 us); M = 37,
+// 1000 -> 2999 19 us with the call (163); M = 1, 14336 -> 20001 INT8 132 us, 2.2 TB/s (5104).
+template <int BITS, bool ZP, int WM, int SC>
+__global__ void __launch_bounds__(THREADS, 2) forward_split_kernel(ForwardArgs p) {
+    constexpr int WN = 4 / WM, TN = 128 * WN;
+    constexpr int TB = BITS == 4 ? 64 : 128;  // byte columns of a wave's tile
+    constexpr int W = TB / 32;                // byte columns a thread converts
+    __shared__ __attribute__((aligned(16))) uint16_t bs[TN * PITCH];
+    const int32_t sp = blockIdx.x % p.splits, tile = blockIdx.x / p.splits;
+    const int32_t m0 = (tile % p.tiles_m) * 32 * WM, j0 = (tile / p.tiles_m) * TB * WN;
+    const int32_t t = threadIdx.x, ln = t & 63, hl = ln >> 5;
+    const int32_t wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int32_t wm = wave % WM, wn = wave / WM;
+    const int32_t begin = sp * p.steps_per_split, end = min(begin + p.steps_per_split, p.steps);
+    const int32_t K = p.K, N = p.N, bpr = p.bpr;
+
+    // This lane's row of a (a row past M repeats the last; its sums are dropped).
+    const int32_t row_a = m0 + 32 * wm;
+    const char* abase = reinterpret_cast<const char*>(p.a + static_cast<size_t>(min(row_a, p.M - 1)) * K);
+    const uint32_t a_off = static_cast<uint32_t>(max(min(ln & 31, p.M - 1 - row_a), 0)) * K * 4u;
+    // The bytes a thread converts: rows 8 rq .. + 7 of the step, W bytes from byte column
+    // j0 + cq W of each tile (past the row's end the last W bytes, shifted into place).
+    const int32_t cq = t & 31, rq = t >> 5;
+    uint32_t w_at[WN], w_shift[WN];
+#pragma unroll
+    for (int i = 0; i < WN; ++i) {
+        const int32_t j = j0 + TB * i + W * cq;
+        w_at[i] = min(j, bpr - W);
+        w_shift[i] = 8 * min(j - static_cast<int32_t>(w_at[i]), W - 1);
+    }
+    // Columns of this lane's sums: block b of the wave's tile.
+    auto column = [&](int32_t lane, int b) {
+        const int32_t j = j0 + TB * wn + W * (lane & 31) + b % W;
+        return BITS == 4 && b >= 2 ? bpr + j : j;
+    };
+    auto exists = [&](int32_t n, int b) { return n < N && (BITS == 8 || b >= 2 || n < bpr); };
+
+    uint32_t w[WN][8], zlo[WN], zhi[WN];
+    float sc[4 / SC][4], sc_next[4 / SC][4];
+    auto load_w = [&](int32_t x) {
+        const int32_t k0 = x * STEP;
+        const char* base = reinterpret_cast<const char*>(p.q) + static_cast<size_t>(k0) * bpr;
+        const size_t zrow = static_cast<size_t>(min(k0 + 8 * rq, K - 1) / p.g) * N;
+#pragma unroll
+        for (int i = 0; i < WN; ++i) {
+#pragma unroll
+            for (int r = 0; r < 8; ++r) {
+                const char* src = base + (static_cast<uint32_t>(min(8 * rq + r, K - 1 - k0)) * bpr + w_at[i]);
+                if constexpr (BITS == 8) w[i][r] = load_any<uint32_t>(src) >> w_shift[i];
+                else w[i][r] = static_cast<uint32_t>(load_any<uint16_t>(src)) >> w_shift[i];
+            }
+            if constexpr (ZP) {
+                const int32_t j = j0 + TB * i + W * cq;
+                const char* zr = reinterpret_cast<const char*>(p.z) + zrow;
+                const int32_t lo = min(j, N - W), hi = min(bpr + j, N - W);
+                if constexpr (BITS == 8) {
+                    zlo[i] = load_any<uint32_t>(zr + lo) >> (8 * min(j - lo, W - 1));
+                } else {
+                    zlo[i] = static_cast<uint32_t>(load_any<uint16_t>(zr + lo)) >> (8 * min(j - lo, W - 1));
+                    zhi[i] = static_cast<uint32_t>(load_any<uint16_t>(zr + hi)) >> (8 * min(bpr + j - hi, W - 1));
+                }
+            }
+        }
+    };
+    auto load_scales = [&](int32_t x, float (&d)[4 / SC][4]) {
+#pragma unroll
+        for (int h = 0; h < 4 / SC; ++h)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const int32_t gi = min(x * STEP + 16 * SC * h, K - 1) / p.g;
+                d[h][b] = p.s[static_cast<size_t>(gi) * N + min(column(ln, b), N - 1)];
+            }
+    };
+    auto convert = [&]() {
+#pragma unroll
+        for (int i = 0; i < WN; ++i)
+            static_for<0, W>([&](auto jc) {
+                constexpr int j = decltype(jc)::value;
+                // byte j of the eight rows minus the zero point, both plus 128
+                auto put = [&](int block, uint32_t zero, auto value) {
+                    const float zf = ZP ? static_cast<float>(zero) : 128.0f;
+                    u32x4 d;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) d[r] = upper_halves(value(w[i][2 * r]) - zf, value(w[i][2 * r + 1]) - zf);
+                    *reinterpret_cast<u32x4*>(bs + (128 * i + 32 * block + cq) * PITCH + 8 * rq) = d;
+                };
+                if constexpr (BITS == 8) {
+                    put(j, ((zlo[i] >> (8 * j)) & 0xFFu) ^ 0x80u, [](uint32_t v) { return ubyte<j>(v ^ 0x80808080u); });
+                } else {
+                    put(j, ((zlo[i] >> (8 * j)) & 0xFFu) ^ 0x80u, [](uint32_t v) { return ubyte<j>((v & 0x0F0Fu) | 0x8080u); });
+                    put(2 + j, ((zhi[i] >> (8 * j)) & 0xFFu) ^ 0x80u, [](uint32_t v) { return ubyte<j>(((v >> 4) & 0x0F0Fu) | 0x8080u); });
+                }
+            });
+    };
+    float a[4][8];
+    auto load_a = [&](int32_t x, int u) {  // a step inside K
+        const char* src = abase + static_cast<int64_t>(x) * (4 * STEP) + (a_off + (64u * u + 32u * hl));
+        const f32x4 v0 = load_any<f32x4>(src), v1 = load_any<f32x4>(src + 16);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            a[u][e] = v0[e];
+            a[u][4 + e] = v1[e];
+        }
+    };
+
+    f32x16 acc[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[b][e] = 0.0f;
+
+    // Products of one step: while the matrix products of 16 k run, the next 16 k of a are
+    // split (and those of step `next` loaded in their place).
+    auto multiply = [&](int32_t next, auto load) {
+        bf16x8 part[2][3], b[2][4];
+        auto prepare = [&](auto uc) {
+            constexpr int u = decltype(uc)::value;
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+                b[u & 1][x] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(
+                                                             bs + (128 * wn + 32 * x + (ln & 31)) * PITCH + 16 * u + 8 * hl));
+            split3(a[u], part[u & 1]);
+            if constexpr (decltype(load)::value) load_a(next, u);
+        };
+        f32x16 sum[4];
+        prepare(std::integral_constant<int, 0>{});
+        __builtin_amdgcn_sched_barrier(0);
+        static_for<0, 4>([&](auto uc) {
+            constexpr int u = decltype(uc)::value;
+            if constexpr (u % SC == 0) {
+#pragma unroll
+                for (int x = 0; x < 4; ++x)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) sum[x][e] = 0.0f;
+            }
+#pragma unroll
+            for (int h = 2; h >= 0; --h)
+#pragma unroll
+                for (int x = 0; x < 4; ++x)
+                    sum[x] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(part[u & 1][h], b[u & 1][x], sum[x], 0, 0, 0);
+            if constexpr (u < 3) {
+                prepare(std::integral_constant<int, u + 1>{});
+                __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+                static_for<0, 12>([&](auto) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+                });
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (u % SC == SC - 1) {
+#pragma unroll
+                for (int x = 0; x < 4; ++x)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) acc[x][e] = fmaf(sc[u / SC][x], sum[x][e], acc[x][e]);
+            }
+        });
+    };
+
+    const int32_t whole = min(end, K / STEP);
+    if (begin < whole) {
+        load_scales(begin, sc);
+        load_w(begin);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) load_a(begin, u);
+        for (int32_t x = begin; x < whole; ++x) {
+            const int32_t next = min(x + 1, whole - 1);
+            __syncthreads();  // the previous step's tile is read
+            convert();
+            __syncthreads();
+            load_w(next);
+            load_scales(next, sc_next);
+            multiply(next, std::true_type{});
+#pragma unroll
+            for (int h = 0; h < 4 / SC; ++h)
+#pragma unroll
+                for (int b = 0; b < 4; ++b) sc[h][b] = sc_next[h][b];
+        }
+    }
+    if (whole < end) {  // K's end: a is zero past it
+        const int32_t x = whole;
+        load_scales(x, sc);
+        load_w(x);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int32_t k = x * STEP + 16 * u + 8 * hl + e;
+                const float v = load_any<float>(abase + (a_off + static_cast<uint32_t>(min(k, K - 1)) * 4u));
+                a[u][e] = k < K ? v : 0.0f;
+            }
+        __syncthreads();
+        convert();
+        __syncthreads();
+        multiply(x, std::false_type{});
+    }
+
+    // Element e of block b: row 8 (e / 4) + 4 hl + e % 4, column column(l, b).
+    const bool direct = p.splits == 1;
+    float* out = p.c + static_cast<size_t>(direct ? 0 : sp) * p.M * N;
+    auto finish = [&](float v, float old, int32_t n) {
+        if (!direct) return v;
+        const float o = fmaf(p.alpha, v, p.accumulate ? old : 0.0f);
+        return p.bias ? o + p.bias[n] : o;
+    };
+    uint64_t nans = 0;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        const int32_t n = column(ln, b);
+        if (!exists(n, b)) continue;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int32_t m = row_a + 8 * (e >> 2) + 4 * hl + (e & 3);
+            if (m >= p.M) continue;
+            float* d = out + static_cast<size_t>(m) * N + n;
+            if (acc[b][e] != acc[b][e]) nans |= uint64_t{1} << (16 * b + e);
+            else *d = finish(acc[b][e], direct && p.accumulate ? *d : 0.0f, n);
+        }
+    }
+    // A NaN may come from splitting an infinity: such an element is summed as
+    // generic_matmul does, term by term.
+    while (nans) {
+        const int32_t i = __builtin_ctzll(nans), b = i >> 4, e = i & 15;
+        nans &= nans - 1;
+        const int32_t m = row_a + 8 * (e >> 2) + 4 * hl + (e & 3), n = column(ln, b);
+        const float* row = p.a + static_cast<size_t>(m) * K;
+        const uint8_t* q = p.q + (BITS == 4 && b >= 2 ? n - bpr : n);
+        float sum = 0.0f;
+        const int32_t k_end = min(end * STEP, K);
+        for (int32_t k1 = begin * STEP; k1 < k_end;) {
+            const int32_t gi = k1 / p.g, k2 = min((gi + 1) * p.g, k_end);
+            float part = 0.0f, rsum = 0.0f;
+            for (; k1 < k2; ++k1) {
+                const int32_t byte = q[static_cast<size_t>(k1) * bpr];
+                const int32_t raw = BITS == 8 ? static_cast<int8_t>(byte) : b >= 2 ? byte >> 4 : byte & 0xF;
+                part = fmaf(row[k1], static_cast<float>(raw), part);
+                rsum += row[k1];
+            }
+            const size_t at = static_cast<size_t>(gi) * N + n;
+            sum = fmaf(p.s[at], fmaf(ZP ? -static_cast<float>(p.z[at]) : -0.0f, rsum, part), sum);
+        }
+        float* d = out + static_cast<size_t>(m) * N + n;
+        *d = finish(sum, direct && p.accumulate ? *d : 0.0f, n);
+    }
+}
+
+// out = (accumulate ? out : 0) + alpha times the slices' sums, in a fixed order (+ bias of
+// rows of N).
 __global__ void __launch_bounds__(THREADS)
     slices_reduce_kernel(const float* __restrict__ part, int32_t splits, int64_t total, float* __restrict__ out,
-                         int32_t accumulate) {
+                         int32_t accumulate, float alpha, const float* __restrict__ bias, int32_t N) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * THREADS + threadIdx.x;
     if (i >= total) return;
     float sum = 0.0f;
@@ -432,7 +703,40 @@ __global__ void __launch_bounds__(THREADS)
         for (int u = 0; u < 8; ++u) v[u] = s0 + u < splits ? part[(s0 + u) * total + i] : 0.0f;
         sum += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
     }
-    out[i] = accumulate ? out[i] + sum : sum;
+    const float o = fmaf(alpha, sum, accumulate ? out[i] : 0.0f);
+    out[i] = bias ? o + bias[i % N] : o;
+}
+
+int32_t launch_slices_reduce(const float* part, int32_t splits, int32_t m, int32_t n, float* out, int32_t accumulate,
+                             float alpha, const float* bias, hipStream_t st) {
+    const int64_t total = static_cast<int64_t>(m) * n, blocks = (total + THREADS - 1) / THREADS;
+    if (blocks > INT32_MAX) return fail(KT_ERR_SHAPE, "grid of %lld blocks is out of range", static_cast<long long>(blocks));
+    slices_reduce_kernel<<<static_cast<uint32_t>(blocks), THREADS, 0, st>>>(part, splits, total, out, accumulate, alpha,
+                                                                          bias, n);
+    KT_LAUNCHED("qmatmul: slices reduce");
+    return KT_OK;
+}
+
+// Slices of `steps` for a grid of `tiles` workgroups: two workgroups per CU, as many slices
+// as the workspace holds (none of it: one slice). slice: bytes of a slice's sums.
+int32_t choose_slices(hipStream_t st, int64_t tiles, int32_t steps, size_t slice, int32_t* per_slice) {
+    int64_t splits = (2 * cu_count() + tiles - 1) / tiles;
+    splits = std::min<int64_t>(std::min<int64_t>(splits, MAX_SPLITS), steps);
+    if (splits > 1 && !workspace_fits(st, splits * slice)) splits = 1;
+    *per_slice = ceil_div(steps, static_cast<int32_t>(splits));
+    return ceil_div(steps, *per_slice);
+}
+
+template <int BITS, bool ZP, int WM>
+void launch_forward_tiles(const ForwardArgs& p, uint32_t blocks, hipStream_t st) {
+    if (p.g % 64 == 0) forward_split_kernel<BITS, ZP, WM, 4><<<blocks, THREADS, 0, st>>>(p);
+    else forward_split_kernel<BITS, ZP, WM, 2><<<blocks, THREADS, 0, st>>>(p);
+}
+template <int BITS, bool ZP>
+void launch_forward_rows(int32_t wm, const ForwardArgs& p, uint32_t blocks, hipStream_t st) {
+    if (wm == 4) launch_forward_tiles<BITS, ZP, 4>(p, blocks, st);
+    else if (wm == 2) launch_forward_tiles<BITS, ZP, 2>(p, blocks, st);
+    else launch_forward_tiles<BITS, ZP, 1>(p, blocks, st);
 }
 
 template <int BITS, int WM>
@@ -466,13 +770,8 @@ int32_t launch_transposed_split(const float* dy, int32_t m, const WeightView& w,
     p.tiles_m = ceil_div(m, 32 * wm);
     const int64_t tiles = static_cast<int64_t>(p.tiles_m) * ceil_div(w.K, 128 * (4 / wm));
     p.steps = ceil_div(w.bpr, w.bits == 4 ? 32 : 64);
-    // Slices of n: two workgroups per CU.
-    int64_t splits = (2 * cu_count() + tiles - 1) / tiles;
-    splits = std::min<int64_t>(std::min<int64_t>(splits, MAX_SPLITS), p.steps);
     const size_t slice = static_cast<size_t>(m) * w.K * sizeof(float);
-    if (splits > 1 && !workspace_fits(st, splits * slice)) splits = 1;
-    p.steps_per_split = ceil_div(p.steps, static_cast<int32_t>(splits));
-    p.splits = ceil_div(p.steps, p.steps_per_split);
+    p.splits = choose_slices(st, tiles, p.steps, slice, &p.steps_per_split);
     // Runs: no longer a sequence of sums than the row-by-row kernel's N / 256, or 16 steps
     // (28 steps in one run at N = 3584 had 1.19e-7 of the 2-norm against its 1.04e-7, two
     // runs of 14 have 1.01e-7; each run after a slice's first takes about 7 us).
@@ -495,13 +794,41 @@ int32_t launch_transposed_split(const float* dy, int32_t m, const WeightView& w,
         : wm == 2 ? launch_transposed_tiles<8, 2>(p, blocks, st)
                   : launch_transposed_tiles<8, 1>(p, blocks, st);
     KT_LAUNCHED("qmatmul_transposed: split kernel");
+    return p.splits > 1 ? launch_slices_reduce(p.out, p.splits, m, w.K, dx, accumulate, 1.0f, nullptr, st) : KT_OK;
+}
+
+// generic_matmul (kt_misc.hip: one thread per output, k in sequence) stays where the product
+// is a few rows of one step (M = 3, 64 -> 70: 10.0 us with the call against 12.8 here; M = 2,
+// 128 -> 100 18.8 against 12.6).
+bool forward_split_preferred(int32_t m, const WeightView& w) {
+    if (w.K <= STEP && m <= 16) return false;
+    // 32 k share a scale, the clamped loads lie in a row; 32-bit lane offsets
+    return w.g % 32 == 0 && w.N >= 8 && w.K <= 1 << 22 && w.bpr <= 1 << 24;
+}
+
+int32_t launch_forward_split(const float* a, int32_t m, const WeightView& w, float* c, int32_t accumulate, float alpha,
+                             const float* bias, hipStream_t st) {
+    ForwardArgs p{a, w.q, w.s, w.z, c, bias, m, w.K, w.N, w.bpr, w.g, w.G, 0, 1, 0, 0, accumulate, alpha};
+    const int32_t wm = m > 64 ? 4 : m > 32 ? 2 : 1;
+    p.tiles_m = ceil_div(m, 32 * wm);
+    const int64_t tiles = static_cast<int64_t>(p.tiles_m) * ceil_div(w.bpr, (w.bits == 4 ? 64 : 128) * (4 / wm));
+    p.steps = ceil_div(w.K, STEP);
+    const size_t slice = static_cast<size_t>(m) * w.N * sizeof(float);
+    p.splits = choose_slices(st, tiles, p.steps, slice, &p.steps_per_split);
     if (p.splits > 1) {
-        const int64_t total = static_cast<int64_t>(m) * w.K;
-        slices_reduce_kernel<<<static_cast<uint32_t>((total + THREADS - 1) / THREADS), THREADS, 0, st>>>(
-            p.out, p.splits, total, dx, accumulate);
-        KT_LAUNCHED("qmatmul_transposed: reduce");
+        void* ws = nullptr;
+        const int32_t status = workspace(st, p.splits * slice, &ws);
+        if (status) return status;
+        p.c = static_cast<float*>(ws);
     }
-    return KT_OK;
+    const int64_t blocks64 = tiles * p.splits;
+    if (blocks64 > INT32_MAX) return fail(KT_ERR_SHAPE, "grid of %lld blocks is out of range", static_cast<long long>(blocks64));
+    const uint32_t blocks = static_cast<uint32_t>(blocks64);
+    if (w.bits == 4) launch_forward_rows<4, true>(wm, p, blocks, st);
+    else if (w.z) launch_forward_rows<8, true>(wm, p, blocks, st);
+    else launch_forward_rows<8, false>(wm, p, blocks, st);
+    KT_LAUNCHED("qmatmul: split kernel");
+    return p.splits > 1 ? launch_slices_reduce(p.c, p.splits, m, w.N, c, accumulate, alpha, bias, st) : KT_OK;
 }
 
 }  // namespace kt

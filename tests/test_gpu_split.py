@@ -61,6 +61,68 @@ def test_transposed_against_64_bits(kt, oracle_lib, m, k, n, bits, g):
     assert same_bits(got, _transposed(kt, dy, qt))
 
 
+# (m, k, n, bits, g, zeros): widths that are not whole quads, row tiles of 32, 64 and 128,
+# column tiles that end in a byte column, steps of 64 k with every kind of end, both scale
+# steps, INT8 with and without zero points
+FORWARD = [
+    (37, 1000, 2999, 4, 64, True), (1, 4096, 1023, 4, 32, True), (2, 4100, 2050, 8, 64, False),
+    (32, 65, 65, 8, 32, True), (33, 63, 515, 8, 64, False), (64, 700, 130, 8, 96, True), (65, 2048, 257, 4, 128, True),
+    (129, 577, 1030, 4, 64, True), (300, 130, 9, 4, 32, True), (150, 9000, 131, 8, 128, False), (16, 14336, 333, 4, 64, True),
+]
+
+
+@pytest.mark.parametrize("m,k,n,bits,g,zeros", FORWARD)
+def test_forward_against_64_bits(kt, oracle_lib, m, k, n, bits, g, zeros):
+    banner("split-forward", m, k, n, bits, g, zeros)
+    q = _weights(oracle_lib, k, n, bits, g, m + k + n)
+    rng = np.random.default_rng(m)
+    if bits == 8 and zeros:
+        q.zeros = rng.integers(-128, 128, q.scales.shape).astype(np.int8)
+    qt = upload_quantized(kt, q)
+    x = (rng.standard_normal((m, k)) * np.exp(4 * rng.standard_normal((m, 1)))).astype(np.float32)
+    w = q.dequantize().astype(np.float64)
+    want = x.astype(np.float64) @ w
+
+    def product(c0=None, alpha=1.0):
+        a = kt.DeviceBuffer.from_numpy(x)
+        c = kt.DeviceBuffer.from_numpy(np.full((m, n), np.nan, np.float32) if c0 is None else c0)
+        kt.MatMul.multiply_quantized(a, qt, c, m, accumulate=c0 is not None, alpha=alpha)
+        kt.synchronize()
+        return c.download(np.float32).reshape(m, n)
+
+    got = product()
+    err = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+    print(f"  largest row error {err.max():.2e}", flush=True)
+    assert err.max() <= TOL
+    c0 = rng.standard_normal((m, n)).astype(np.float32)
+    assert normwise_rel(product(c0, -0.5), c0 - 0.5 * want) <= TOL
+    assert same_bits(got, product())
+
+
+def test_forward_infinities_and_nans(kt, oracle_lib):
+    """An infinite or NaN input reaches its row alone, whose outputs are those of the group
+    sums scale (sum a raw - zero sum a): none finite (a NaN where zero sum a is one)."""
+    m, k, n = 40, 700, 333
+    banner("split-forward-inf")
+    for bits in (4, 8):
+        q = _weights(oracle_lib, k, n, bits, 64, 15)
+        qt = upload_quantized(kt, q)
+        x = np.random.default_rng(16).standard_normal((m, k)).astype(np.float32)
+
+        def product(v):
+            a, c = kt.DeviceBuffer.from_numpy(v), kt.DeviceBuffer(m * n * 4)
+            kt.MatMul.multiply_quantized(a, qt, c, m, accumulate=False)
+            kt.synchronize()
+            return c.download(np.float32).reshape(m, n)
+
+        plain, odd = product(x), x.copy()
+        odd[3, 17], odd[20, 699], odd[21, 500] = np.inf, -np.inf, np.nan
+        got = product(odd)
+        rest = np.setdiff1d(np.arange(m), [3, 20, 21])
+        assert same_bits(got[rest], plain[rest])
+        assert np.isnan(got[21]).all() and not np.isfinite(got[[3, 20]]).any()
+
+
 def test_transposed_infinities_and_nans(kt, oracle_lib):
     """An infinite or NaN dY element reaches its row alone, with the products' signs; finite
     elements next to it, also the largest fp32 numbers, stay exact."""
