@@ -24,7 +24,10 @@
 // differ from the reference's sequential sums by fp32 rounding only.
 #include <math.h>
 
+#include <atomic>
+
 #include "kt_common.h"
+#include "kt_split.h"
 
 namespace kt {
 namespace {
@@ -627,36 +630,80 @@ __global__ void __launch_bounds__(THREADS) attention_kernel(AttnArgs a) {
     }
 }
 
-// ---- prefill attention: blocked over queries, fp32 MFMA ---------------------------------
-// Workgroup (kv head g, block of QB = 128 / G consecutive tokens): the query rows
-// r = (token t0 + r / G, head g G + r % G), r < QB G, over keys 0 .. position + token,
-// 64 keys at a time; K and V tiles in LDS serve the four waves (32 rows each), so a key
-// row is read once per workgroup instead of once per token. Both products run on
-// v_mfma_f32_32x32x2_f32 (fp32 operands, fp32 sums; the reference's arithmetic up to
-// summation order):
+// ---- prefill attention: blocked over queries, fp32 precision on the bf16 matrix units -----
+// Workgroup (kv head g, block of 64 / G consecutive tokens): the query rows
+// r = (token t0 + r / G, head g G + r % G), r < 64, over keys 0 .. position + token, 64 keys
+// at a time. Wave w takes rows 32 (w % 2) .. + 31 and keys 32 (w / 2) .. + 31 of every tile;
+// the two key halves of a row meet at the end, through LDS.
+// An fp32 number is the exact sum of three bf16 numbers (kt_split.h); the product of two is
+// taken as the six products of parts down to 2^-16 of the largest (the three left out are
+// below an fp32 rounding), on v_mfma_f32_32x32x16_bf16 with fp32 sums, small products first:
+// 2.7 times the rate of the fp32 matrix instruction.
 //   S^T = K Q^T: lane l ends with the scores of query row l % 32 against the 16 keys
-//     8 (e / 4) + 4 (l / 32) + e % 4 of each 32-key block (register e), so the running
-//     maximum, the exponentials and the rescaling of a row stay inside lanes l, l ^ 32;
-//   O^T += V^T P^T, taking the keys of each block in that same order: the B operand of
-//     step e is register e of the scores, as they lie.
-// Blocks go out longest first (the last tokens see the most keys).
-constexpr int PQ_ROWS = 128;  // query rows per workgroup
+//     8 (e / 4) + 4 (l / 32) + e % 4 of the wave's 32 (register e), so the running maximum,
+//     the exponentials and the rescaling of a row stay inside lanes l, l ^ 32. Q is scaled
+//     by log2(e) / sqrt(head_dim) before it is split: the exponentials are v_exp_f32 of a
+//     difference.
+//   O^T += V^T P^T, taking the keys in that same order: V lies transposed in LDS with the
+//     eight keys of a lane's operand side by side. A tile's sum starts from zero and joins
+//     the rescaled running sum with one multiply-add.
+// The longest blocks go out first, the shortest with them while two workgroups per CU hold
+// all (workgroups y and y + 32 of an XCD share a CU: the pair is then about as long as any).
+// 1024 tokens, 32 query and 8 kv heads of 64: 44 us (fp32 matrix instructions on 128 rows a
+// workgroup: 103 us), head dimension 128 119 us (184), 64 tokens after 1024 44 us (107);
+// error against 64 bits 1.4e-7 (3.3e-7). Bound by the longest block's chain of tiles: about
+// 565 vector instructions and 48 matrix products a wave and tile, which overlap only where
+// two workgroups share the CU.
+constexpr int PQ_ROWS = 64;   // query rows per workgroup
 constexpr int PKT = 64;       // keys per tile
 constexpr int PREFILL_MIN_TOKENS = 16;  // fewer tokens: the per-token kernel with key splits
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float v4f __attribute__((ext_vector_type(4)));
 
 template <int HD>
-__global__ void __launch_bounds__(THREADS) attention_prefill_kernel(AttnArgs a, int32_t tokens, int32_t qb_tokens,
-                                                                    int32_t nqb) {
-    extern __shared__ float smem[];
-    constexpr int KP = HD + 1;  // K row stride: 32 lanes on 32 rows hit distinct banks
-    constexpr int VP = HD + 8;  // V row stride: the two half-waves read rows 4 apart on other banks
-    constexpr int DB = HD / 32;
-    constexpr int QS = HD / 2;
-    constexpr int TF = PKT * HD / 4 / THREADS;  // float4 of a K (V) tile per thread
-    const int32_t g = blockIdx.x;
-    const int32_t qb = nqb - 1 - static_cast<int32_t>(blockIdx.y);
+struct PrefillShared {
+    uint16_t k[3][PKT][HD + 8];   // parts of the keys (row strides of 16 bytes times an odd number)
+    uint16_t v[3][HD][PKT + 8];   // parts of the values, transposed, keys in operand order
+};
+
+// One query row as a single wave sums it in fp32, for a row whose result is not a number:
+// splitting an infinity makes NaNs, so such rows are computed from the fp32 values.
+template <int HD>
+__device__ __forceinline__ void attend_row(const AttnArgs& a, const float* q, size_t base, int32_t keys, float* dst,
+                                           float* p_s) {
+    const int32_t ln = threadIdx.x & 63;
+    auto score = [&](int32_t j) {
+        const float* k = a.ck + (base + j) * HD;
+        float s = 0.0f;
+        for (int32_t d = 0; d < HD; ++d) s = fmaf(q[d], k[d], s);
+        return s * a.scale;
+    };
+    float m = -INFINITY;
+    for (int32_t j = ln; j < keys; j += 64) m = fmaxf(m, score(j));
+    m = wave_max_dpp(m);
+    float l = 0.0f, o[HD / 64];
+    for (int i = 0; i < HD / 64; ++i) o[i] = 0.0f;
+    for (int32_t j0 = 0; j0 < keys; j0 += 64) {
+        const float p = j0 + ln < keys ? expf(score(j0 + ln) - m) : 0.0f;
+        l += wave_sum_dpp(p);
+        p_s[ln] = p;
+        __builtin_amdgcn_wave_barrier();
+        for (int32_t j = 0; j < min(64, keys - j0); ++j)
+            for (int i = 0; i < HD / 64; ++i) o[i] = fmaf(p_s[j], a.cv[(base + j0 + j) * HD + ln + 64 * i], o[i]);
+        __builtin_amdgcn_wave_barrier();
+    }
+    for (int i = 0; i < HD / 64; ++i) dst[ln + 64 * i] = o[i] * (1.0f / l);
+}
+
+template <int HD>
+__global__ void __launch_bounds__(THREADS, HD == 64 ? 2 : 1)
+    attention_prefill_kernel(AttnArgs a, int32_t tokens, int32_t qb_tokens, int32_t nqb, int32_t paired) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t prefill_smem[];
+    PrefillShared<HD>& sh = *reinterpret_cast<PrefillShared<HD>*>(prefill_smem);
+    constexpr int DB = HD / 32;               // 32-dim blocks of the output
+    constexpr int QS = HD / 16;               // 16-dim steps of a score
+    constexpr int NI = PKT * HD / 8 / THREADS;  // groups of eight K (V) values a thread stages
+    const int32_t g = blockIdx.x, y = blockIdx.y;
+    const int32_t half_y = (nqb + 1) / 2;
+    const int32_t qb = paired && y >= half_y ? y - half_y : nqb - 1 - y;
     const int32_t G = a.num_heads / a.num_kv_heads;
     const int32_t dim = a.num_heads * HD;
     const int32_t t0 = qb * qb_tokens;
@@ -664,154 +711,207 @@ __global__ void __launch_bounds__(THREADS) attention_prefill_kernel(AttnArgs a, 
     const int32_t P0 = *a.position;
     const int32_t n_keys = min(P0 + t_end, a.max_seq);  // never read outside the cache
     const size_t base = (static_cast<size_t>(a.layer) * a.num_kv_heads + g) * a.max_seq;  // row of key 0
-    const int32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int32_t rl = lane & 31, h = lane >> 5;
+    const int32_t tid = threadIdx.x, lane = tid & 63, hl = lane >> 5;
+    const int32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), rb = wave & 1, kh = wave >> 1;
 
-    const int32_t r = wave * 32 + rl;  // this lane's query row
-    const int32_t tl = r / G;
-    const int32_t tok = t0 + tl;
+    const int32_t r = rb * 32 + (lane & 31);  // this lane's query row
+    const int32_t tl = r / G, tok = t0 + tl;
     const bool row_ok = tl < qb_tokens && tok < t_end;
     const int32_t head = g * G + r % G;
     const int32_t p_r = row_ok ? min(P0 + tok, a.max_seq - 1) : -1;  // last key of the row
+    const float* qrow = a.q + static_cast<size_t>(min(tok, tokens - 1)) * dim + head * HD;
 
-    // the query rows through LDS into each lane's MFMA fragment: Q[r][2 s + h]
-    float qf[QS];
-    {
-        float* qs = smem;  // [PQ_ROWS][KP]
-        for (int32_t e = tid; e < PQ_ROWS * HD / 4; e += THREADS) {
-            const int32_t rr = e / (HD / 4), c4 = e % (HD / 4);
-            const int32_t tt = t0 + rr / G;
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (rr / G < qb_tokens && tt < t_end)
-                v = *reinterpret_cast<const float4*>(a.q + static_cast<size_t>(tt) * dim + (g * G + rr % G) * HD + 4 * c4);
-            float* d = qs + rr * KP + 4 * c4;
-            d[0] = v.x;
-            d[1] = v.y;
-            d[2] = v.z;
-            d[3] = v.w;
-        }
-        __syncthreads();
+    // the row's parts as the products' second operand: dims 16 s + 8 hl .. + 7
+    bf16x8 qp[QS][3];
+    const float qscale = a.scale * 1.4426950408889634f;
 #pragma unroll
-        for (int s = 0; s < QS; ++s) qf[s] = qs[r * KP + 2 * s + h];
-        __syncthreads();  // the area becomes the K and V tiles
+    for (int s = 0; s < QS; ++s) {
+        const f4* src = reinterpret_cast<const f4*>(qrow + 16 * s + 8 * hl);
+        const f4 v0 = src[0], v1 = src[1];
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[e] = v0[e] * qscale;
+            v[4 + e] = v1[e] * qscale;
+        }
+        split3(v, qp[s]);
     }
+    // rows of the wave: the first and last key any of them sees last
+    int32_t p_min = row_ok ? p_r : 0x7FFFFFFF, p_max = p_r;
+#pragma unroll
+    for (int o = 16; o > 0; o >>= 1) {
+        p_min = min(p_min, __shfl_xor(p_min, o));
+        p_max = max(p_max, __shfl_xor(p_max, o));
+    }
+    p_min = __builtin_amdgcn_readfirstlane(p_min);
+    p_max = __builtin_amdgcn_readfirstlane(p_max);
 
-    float* ks = smem;             // [PKT][KP]
-    float* vs = smem + PKT * KP;  // [PKT][VP]
+    // A tile's values, eight a group: of K dims 8 o .. + 7 of a key; of V one dim of the eight
+    // keys of an operand (octet o of the tile: keys 32 (o / 4) + 16 ((o / 2) % 2) + 4 (o % 2)
+    // + {0 .. 3, 8 .. 11}). Rows past n_keys repeat the last key and are masked.
+    float kr[NI][8], vr[NI][8];
+    auto load_tile = [&](int32_t k0) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int32_t e = tid + i * THREADS;
+            const f4* src = reinterpret_cast<const f4*>(a.ck + (base + min(k0 + e / (HD / 8), n_keys - 1)) * HD + 8 * (e % (HD / 8)));
+            const f4 v0 = src[0], v1 = src[1];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                kr[i][u] = v0[u];
+                kr[i][4 + u] = v1[u];
+            }
+            const int32_t d = e % HD, o = e / HD;
+            const int32_t key = k0 + 32 * (o >> 2) + 16 * ((o >> 1) & 1) + 4 * (o & 1);
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                vr[i][u] = a.cv[(base + min(key + (u & 3) + 8 * (u >> 2), n_keys - 1)) * HD + d];
+        }
+    };
+    auto store_tile = [&]() {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int32_t e = tid + i * THREADS;
+            bf16x8 part[3];
+            split3(kr[i], part);
+#pragma unroll
+            for (int h = 0; h < 3; ++h)
+                *reinterpret_cast<bf16x8*>(&sh.k[h][e / (HD / 8)][8 * (e % (HD / 8))]) = part[h];
+            split3(vr[i], part);
+#pragma unroll
+            for (int h = 0; h < 3; ++h) *reinterpret_cast<bf16x8*>(&sh.v[h][e % HD][8 * (e / HD)]) = part[h];
+        }
+    };
+
     f32x16 oacc[DB];
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
         for (int e = 0; e < 16; ++e) oacc[db][e] = 0.0f;
-    float m = -INFINITY, l = 0.0f;
+    float m = -INFINITY, l = 0.0f;  // the row's running maximum (in powers of two), this lane's sum
 
-    // a tile's K and V rows, all loads out before the first is used; rows past n_keys
-    // repeat the last key and are masked, and the tile after the last one repeats it
-    // (unconditional loads: no branch, and the arrays stay in registers)
-    v4f kr[TF], vr[TF];  // (native vectors: the HIP float4 struct keeps the arrays in scratch)
+    auto attend_tile = [&](int32_t k0) {  // the wave's 32 keys from k0
+        f32x16 big, small;
 #pragma unroll
-    for (int i = 0; i < TF; ++i) {
-        const int32_t e = tid + i * THREADS;
-        const int32_t j = e / (HD / 4), c4 = e % (HD / 4);
-        const size_t row = base + min(j, n_keys - 1);
-        kr[i] = *reinterpret_cast<const v4f*>(a.ck + row * HD + 4 * c4);
-        vr[i] = *reinterpret_cast<const v4f*>(a.cv + row * HD + 4 * c4);
-    }
-    for (int32_t k0 = 0; k0 < n_keys; k0 += PKT) {
+        for (int e = 0; e < 16; ++e) big[e] = small[e] = 0.0f;
 #pragma unroll
-        for (int i = 0; i < TF; ++i) {
-            const int32_t e = tid + i * THREADS;
-            const int32_t j = e / (HD / 4), c4 = e % (HD / 4);
-            float* kd = ks + j * KP + 4 * c4;
-            kd[0] = kr[i][0];
-            kd[1] = kr[i][1];
-            kd[2] = kr[i][2];
-            kd[3] = kr[i][3];
-            *reinterpret_cast<v4f*>(vs + j * VP + 4 * c4) = vr[i];
+        for (int s = 0; s < QS; ++s) {
+            bf16x8 kp[3];
+#pragma unroll
+            for (int h = 0; h < 3; ++h)
+                kp[h] = *reinterpret_cast<const bf16x8*>(&sh.k[h][32 * kh + (lane & 31)][16 * s + 8 * hl]);
+            small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kp[2], qp[s][0], small, 0, 0, 0);
+            small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kp[0], qp[s][2], small, 0, 0, 0);
+            small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kp[1], qp[s][1], small, 0, 0, 0);
+            small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kp[1], qp[s][0], small, 0, 0, 0);
+            small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kp[0], qp[s][1], small, 0, 0, 0);
+            big = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kp[0], qp[s][0], big, 0, 0, 0);
         }
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < TF; ++i) {
-            const int32_t e = tid + i * THREADS;
-            const int32_t j = e / (HD / 4), c4 = e % (HD / 4);
-            const size_t row = base + min(k0 + PKT + j, n_keys - 1);
-            kr[i] = *reinterpret_cast<const v4f*>(a.ck + row * HD + 4 * c4);
-            vr[i] = *reinterpret_cast<const v4f*>(a.cv + row * HD + 4 * c4);
-        }
-
-        // S^T = K Q^T for the two 32-key blocks
-        f32x16 sacc[2];
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-#pragma unroll
-            for (int e = 0; e < 16; ++e) sacc[kb][e] = 0.0f;
-#pragma unroll
-            for (int s = 0; s < QS; ++s)
-                sacc[kb] = __builtin_amdgcn_mfma_f32_32x32x2f32(ks[(kb * 32 + rl) * KP + 2 * s + h], qf[s], sacc[kb], 0,
-                                                                0, 0);
-        }
-        // scale, causal mask, running max and sum of the row (lanes l and l ^ 32)
+        float p[16];
         float tmax = -INFINITY;
+        const bool masked = k0 + 31 > p_min;
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int32_t j = k0 + kb * 32 + 8 * (e >> 2) + 4 * h + (e & 3);
-                const float v = j <= p_r ? sacc[kb][e] * a.scale : -INFINITY;
-                sacc[kb][e] = v;
-                tmax = fmaxf(tmax, v);
-            }
+        for (int e = 0; e < 16; ++e) {
+            p[e] = big[e] + small[e];
+            if (masked) p[e] = k0 + 8 * (e >> 2) + 4 * hl + (e & 3) <= p_r ? p[e] : -INFINITY;
+            tmax = fmaxf(tmax, p[e]);
+        }
         tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
         const float m_new = fmaxf(m, tmax);
-        const bool none = m_new == -INFINITY;  // no key of the row yet (a padding row)
-        const float alpha = none || m == -INFINITY ? (none ? 1.0f : 0.0f) : expf(m - m_new);
+        const float m_use = m_new == -INFINITY ? 0.0f : m_new;  // no key of the row yet
+        const float alpha = __builtin_amdgcn_exp2f(m - m_use);
         float psum = 0.0f;
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const float p = none ? 0.0f : expf(sacc[kb][e] - m_new);
-                sacc[kb][e] = p;
-                psum += p;
-            }
-        psum += __shfl_xor(psum, 32);
+        for (int e = 0; e < 16; ++e) {
+            p[e] = __builtin_amdgcn_exp2f(p[e] - m_use);
+            psum += p[e];
+        }
         l = l * alpha + psum;
         m = m_new;
+        bf16x8 pp[2][3];
 #pragma unroll
-        for (int db = 0; db < DB; ++db)
+        for (int st = 0; st < 2; ++st) {
+            float v[8];
 #pragma unroll
-            for (int e = 0; e < 16; ++e) oacc[db][e] *= alpha;
-        // O^T += V^T P^T, the keys of block kb in the order of the score registers
+            for (int e = 0; e < 8; ++e) v[e] = p[8 * st + e];
+            split3(v, pp[st]);
+        }
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
+        for (int db = 0; db < DB; ++db) {
+            f32x16 sum;
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const float* vrow = vs + (kb * 32 + 8 * (e >> 2) + 4 * h + (e & 3)) * VP + rl;
+            for (int e = 0; e < 16; ++e) sum[e] = 0.0f;
+            bf16x8 vp[2][3];
 #pragma unroll
-                for (int db = 0; db < DB; ++db)
-                    oacc[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[db * 32], sacc[kb][e], oacc[db], 0, 0, 0);
+            for (int st = 0; st < 2; ++st) {
+#pragma unroll
+                for (int h = 0; h < 3; ++h)
+                    vp[st][h] = *reinterpret_cast<const bf16x8*>(&sh.v[h][32 * db + (lane & 31)][32 * kh + 16 * st + 8 * hl]);
+                sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vp[st][2], pp[st][0], sum, 0, 0, 0);
+                sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vp[st][0], pp[st][2], sum, 0, 0, 0);
+                sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vp[st][1], pp[st][1], sum, 0, 0, 0);
+                sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vp[st][1], pp[st][0], sum, 0, 0, 0);
+                sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vp[st][0], pp[st][1], sum, 0, 0, 0);
             }
-        __syncthreads();  // the tiles are read before the next store
-    }
+#pragma unroll
+            for (int st = 0; st < 2; ++st) sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vp[st][0], pp[st][0], sum, 0, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 16; ++e) oacc[db][e] = fmaf(oacc[db][e], alpha, sum[e]);
+        }
+    };
 
-    // O^T element (d, r) of block db: lane r + 32 ((d / 4) % 2), register (d / 8) * 4 + d % 4
-    if (row_ok) {
-        const float inv = 1.0f / l;
-        float* dst = a.context + static_cast<size_t>(tok) * dim + head * HD;
+    load_tile(0);
+    for (int32_t k0 = 0; k0 < n_keys; k0 += PKT) {
+        store_tile();
+        __syncthreads();
+        load_tile(k0 + PKT);  // (past the end the last key again, unused)
+        if (k0 + 32 * kh <= p_max) attend_tile(k0 + 32 * kh);
+        __syncthreads();  // the tile is read before the next store
+    }
+    l += __shfl_xor(l, 32);
+
+    // The second half's (sums, maximum, sum of exponentials) through LDS to the first's wave.
+    // O^T element (d, r) of block db: lane r + 32 ((d / 4) % 2), register (d / 8) * 4 + d % 4.
+    float* ex = reinterpret_cast<float*>(prefill_smem) + rb * (DB * 16 + 2) * 64 + lane;
+    if (kh == 1) {
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
-            for (int c = 0; c < 4; ++c)
-                *reinterpret_cast<float4*>(dst + db * 32 + 8 * c + 4 * h) =
-                    make_float4(oacc[db][4 * c] * inv, oacc[db][4 * c + 1] * inv, oacc[db][4 * c + 2] * inv,
-                                oacc[db][4 * c + 3] * inv);
+            for (int e = 0; e < 16; ++e) ex[(db * 16 + e) * 64] = oacc[db][e];
+        ex[DB * 16 * 64] = m;
+        ex[(DB * 16 + 1) * 64] = l;
     }
-}
-
-size_t attention_prefill_lds(int32_t head_dim) {
-    const size_t q = static_cast<size_t>(PQ_ROWS) * (head_dim + 1);
-    const size_t kv = static_cast<size_t>(PKT) * (head_dim + 1) + static_cast<size_t>(PKT) * (head_dim + 8);
-    return (q > kv ? q : kv) * sizeof(float);
+    __syncthreads();
+    if (kh == 1) return;
+    const float m1 = ex[DB * 16 * 64], l1 = ex[(DB * 16 + 1) * 64];
+    const float mx = fmaxf(m, m1);
+    const float m_use = mx == -INFINITY ? 0.0f : mx;
+    const float w0 = __builtin_amdgcn_exp2f(m - m_use), w1 = __builtin_amdgcn_exp2f(m1 - m_use);
+    const float inv = 1.0f / (l * w0 + l1 * w1);
+    float* dst = a.context + static_cast<size_t>(min(tok, tokens - 1)) * dim + head * HD;
+    bool nan = false;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            f4 o;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                o[i] = (oacc[db][4 * c + i] * w0 + ex[(db * 16 + 4 * c + i) * 64] * w1) * inv;
+                nan = nan || o[i] != o[i];
+            }
+            if (row_ok) *reinterpret_cast<f4*>(dst + db * 32 + 8 * c + 4 * hl) = o;
+        }
+    uint64_t rows = __ballot(nan && row_ok);
+    rows = (rows | rows >> 32) & 0xFFFFFFFFull;
+    while (rows) {
+        const int32_t rr = rb * 32 + __builtin_ctzll(rows), tt = t0 + rr / G, hh = g * G + rr % G;
+        rows &= rows - 1;
+        const size_t at = static_cast<size_t>(tt) * dim + hh * HD;
+        // (this wave's own part of the exchange area; the other row block's wave may still read its own)
+        attend_row<HD>(a, a.q + at, base, min(P0 + tt, a.max_seq - 1) + 1, a.context + at,
+                       reinterpret_cast<float*>(prefill_smem) + rb * (DB * 16 + 2) * 64);
+    }
 }
 
 // ---- SwiGLU gate -----------------------------------------------------------------------
@@ -1041,17 +1141,18 @@ static int32_t attention_launch(const float* q, int32_t tokens, const int32_t* p
         const int32_t qb_tokens = PQ_ROWS / G;
         const int32_t nqb = ceil_div(tokens, qb_tokens);
         const dim3 grid(static_cast<uint32_t>(num_kv_heads), static_cast<uint32_t>(nqb));
-        const size_t lds = attention_prefill_lds(head_dim);
+        const int32_t paired = static_cast<int64_t>(num_kv_heads) * nqb <= 2 * cu_count();
         if (head_dim == 64) {
-            attention_prefill_kernel<64><<<grid, THREADS, lds, st>>>(a, tokens, qb_tokens, nqb);
+            attention_prefill_kernel<64><<<grid, THREADS, sizeof(PrefillShared<64>), st>>>(a, tokens, qb_tokens, nqb, paired);
         } else {
-            static bool raised = false;
+            static std::atomic<bool> raised{false};
             if (!raised) {  // beyond the default dynamic LDS limit (160 KB per CU on gfx950)
                 KT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_prefill_kernel<128>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, 160 << 10));
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, sizeof(PrefillShared<128>)));
                 raised = true;
             }
-            attention_prefill_kernel<128><<<grid, THREADS, lds, st>>>(a, tokens, qb_tokens, nqb);
+            attention_prefill_kernel<128><<<grid, THREADS, sizeof(PrefillShared<128>), st>>>(a, tokens, qb_tokens, nqb,
+                                                                                          paired);
         }
         KT_LAUNCHED("prefill attention kernel");
         return KT_OK;

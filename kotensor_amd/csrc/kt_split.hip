@@ -18,14 +18,12 @@
 
 #include "kt_common.h"
 #include "kt_packed.h"
+#include "kt_split.h"
 
 namespace kt {
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int THREADS = 256;
 constexpr int STEP = 64;          // elements of the summed dimension per step
@@ -44,33 +42,6 @@ __device__ __forceinline__ T load_any(const void* p) {
 __device__ __forceinline__ uint32_t load_end(const void* row, int32_t i, int32_t bytes) {
     const int32_t at = min(i, bytes - 4);
     return load_any<uint32_t>(static_cast<const uint8_t*>(row) + at) >> (8 * min(i - at, 3));
-}
-
-// The upper halves of two floats in one dword: their bf16 truncations.
-__device__ __forceinline__ uint32_t upper_halves(float lo, float hi) {
-    return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, hi), __builtin_bit_cast(uint32_t, lo), 0x07060302u);
-}
-// v minus its bf16 truncation, exact. (One v_dot2_f32_bf16 does the same, but runs on the
-// matrix unit: four of them beside a 32x32x16 product took 63 cycles, four multiply-adds 38.)
-__device__ __forceinline__ float below_upper(float v) {
-    return v - __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v) & 0xFFFF0000u);
-}
-
-// Eight finite fp32 numbers as three bf16 operands, p = part[0] + part[1] + part[2]. An
-// infinity makes a NaN of its lower parts; the callers look for NaN sums.
-__device__ __forceinline__ void split3(const float (&p)[8], bf16x8 (&part)[3]) {
-    u32x4 h, m, l;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float a = p[2 * i], b = p[2 * i + 1];
-        h[i] = upper_halves(a, b);
-        const float ra = below_upper(a), rb = below_upper(b);
-        m[i] = upper_halves(ra, rb);
-        l[i] = upper_halves(below_upper(ra), below_upper(rb));
-    }
-    part[0] = __builtin_bit_cast(bf16x8, h);
-    part[1] = __builtin_bit_cast(bf16x8, m);
-    part[2] = __builtin_bit_cast(bf16x8, l);
 }
 
 template <int I>

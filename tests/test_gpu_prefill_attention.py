@@ -1,0 +1,82 @@
+"""The prefill attention (kt_decoder.hip, fp32 precision by products of bf16 parts) against
+64 bits: blocks of 64 query rows that end inside a token's heads, tiles of 64 keys with
+every kind of end, a wave without keys of its own, both orders of the blocks, both head
+dimensions; and rows with infinities.
+
+Bound: six products of parts per element leave an fp32 rounding each; with the fp32 sums of
+up to 1600 keys and the exponential's rounding the result is held to 1e-6 normwise."""
+import numpy as np
+import pytest
+
+from conftest import normwise_rel
+from gpu_helpers import banner
+
+pytestmark = pytest.mark.gpu
+
+
+def _call(kt, q, keys, values, start, heads):
+    from kotensor_amd import _lib
+    kvh, max_seq, d = keys.shape
+    tokens = q.shape[0]
+    dq, dk, dv = (kt.DeviceBuffer.from_numpy(a) for a in (q, keys, values))
+    pos, out = kt.DeviceBuffer.from_numpy(np.array([start], np.int32)), kt.DeviceBuffer(q.nbytes)
+    _lib.call("kt_attention", dq.ptr, tokens, pos.ptr, start + tokens, dk.ptr, dv.ptr, 0, max_seq, heads, kvh, d, out.ptr, None)
+    kt.synchronize()
+    return out.download(np.float32).reshape(q.shape)
+
+
+def _exact(q, keys, values, start, heads):
+    kvh, _, d = keys.shape
+    tokens = q.shape[0]
+    out = np.empty(q.shape)
+    visible = np.arange(start + tokens)[None] <= start + np.arange(tokens)[:, None]
+    for h in range(heads):
+        k, v = (a[h // (heads // kvh), :start + tokens].astype(np.float64) for a in (keys, values))
+        s = q[:, h * d:(h + 1) * d].astype(np.float64) @ k.T / np.sqrt(d)
+        p = np.where(visible, np.exp(s - np.where(visible, s, -np.inf).max(1, keepdims=True)), 0.0)
+        out[:, h * d:(h + 1) * d] = p @ v / p.sum(1, keepdims=True)
+    return out
+
+
+@pytest.mark.parametrize("tokens,start,heads,kvh,d", [
+    (16, 0, 4, 4, 64), (17, 47, 14, 2, 64), (64, 0, 32, 8, 64), (65, 63, 8, 1, 64), (100, 1500, 4, 1, 64),
+    (700, 1, 8, 8, 64), (16, 0, 8, 8, 128), (33, 95, 16, 2, 128), (130, 200, 7, 1, 128), (40, 3, 3, 1, 64),
+])
+def test_prefill_attention_against_64_bits(kt, tokens, start, heads, kvh, d):
+    banner("prefill-attention", tokens, start, heads, kvh, d)
+    rng = np.random.default_rng(tokens + start)
+    max_seq = start + tokens + 5
+    q = (2.0 * rng.standard_normal((tokens, heads * d))).astype(np.float32)
+    keys, values = (rng.standard_normal((kvh, max_seq, d)).astype(np.float32) for _ in range(2))
+    keys[:, start + tokens:] = np.nan  # past the last key: never used
+    err = normwise_rel(_call(kt, q, keys, values, start, heads), _exact(q, keys, values, start, heads))
+    print(f"  error {err:.2e}", flush=True)
+    assert err <= 1e-6
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_prefill_attention_infinities(kt, d):
+    """A key whose score is minus infinity adds nothing, an infinite value makes infinities
+    of the rows that see it, a NaN query NaNs of its own row; other rows keep their values."""
+    tokens, heads, kvh = 70, 4, 2
+    rng = np.random.default_rng(7)
+    q = rng.standard_normal((tokens, heads * d)).astype(np.float32)
+    q[:, ::d] = np.abs(q[:, ::d]) + 0.1  # each head's first dim positive
+    keys, values = (rng.standard_normal((kvh, tokens, d)).astype(np.float32) for _ in range(2))
+    want = _exact(q, keys, values, 0, heads)
+    keys[0, 5] = 0.0
+    keys[0, 5, 0] = -np.inf
+    values[1, 60, 3] = np.inf
+    q[20, 2 * d + 1] = np.nan
+    banner("prefill-attention-inf", d)
+    got = _call(kt, q, keys, values, 0, heads)
+    plain = keys.copy()
+    plain[0, 5, 0] = -1e6  # the same weights: nothing
+    ref = _exact(q, plain, np.where(np.isinf(values), 0.0, values).astype(np.float32), 0, heads)
+    g0, r0 = got[:, :2 * d], ref[:, :2 * d]
+    assert normwise_rel(np.delete(g0, 5, 0), np.delete(r0, 5, 0)) <= 1e-6 and np.isfinite(g0).all()
+    third = got[:, 2 * d:3 * d]
+    assert np.isnan(third[20]).all()
+    assert np.isposinf(third[60:, 3]).all()
+    keep = np.setdiff1d(np.arange(60), [20])
+    assert normwise_rel(third[keep], want[keep, 2 * d:3 * d]) <= 1e-6
