@@ -219,4 +219,6 @@ def check(status: int, what: str = "") -> None:
 
 def call(name: str, *args) -> None:
     """Calls an entry point and raises on a non-zero status."""
-    check(getattr(lib(), name)(*args), name)
+    status = getattr(_lib or _load(), name)(*args)
+    if status:
+        check(status, name)

@@ -9,7 +9,7 @@ import numpy as np
 
 from . import _lib
 from .device import DeviceBuffer, Stream, default_stream
-from .matmul import DeviceTensor
+from .matmul import DeviceTensor, _call_group
 from .quantization import Quantization, QuantizedTensor
 
 
@@ -72,16 +72,17 @@ class QuantizedLinear:
 def forward_into_group(layers, x: DeviceTensor, outs, stream: Stream | None = None):
     """``outs[i] = x · deq(layers[i].weight) + layers[i].bias`` for projections of one input
     (wQ/wK/wV, Attention.kt:220-222; wGate/wUp, SwiGLU.kt:19-25), one launch per four layers."""
-    from .matmul import MatMul
-
     m, k = x.shape
     for layer, out in zip(layers, outs):
         if layer.in_size != k:
             raise _lib.IllegalArgumentException(f"{k} != {layer.in_size}")
         if out.shape != (m, layer.out_size):
             raise _lib.IllegalArgumentException(f"out shape {list(out.shape)} != [{m}, {layer.out_size}]")
-    MatMul.multiply_quantized_group(x, [l.weight for l in layers], outs, m, accumulate=False, alpha=1.0,
-                                    biases=[l.bias for l in layers], stream=stream)
+    if len(layers) != len(outs):
+        raise _lib.IllegalArgumentException("weights, outputs and biases differ in length")
+    if layers:  # (a tensor's buffer holds its shape: nothing more to check)
+        _call_group(x.buffer._ptr, m, [l._weight._struct for l in layers], [o.buffer._ptr for o in outs],
+                    [None if l.bias is None else l.bias.buffer._ptr for l in layers], 0, 1.0, stream)
     return outs
 
 

@@ -83,6 +83,14 @@ def _nbytes(x):
     return None
 
 
+def _call_group(a, m: int, structs, outputs, biases, accumulate: int, alpha: float, stream: Stream | None) -> None:
+    """kt_qmatmul_group on checked operands: kt_qweight structs, output and bias addresses."""
+    count = len(structs)
+    pointers = ctypes.c_void_p * count
+    _lib.call("kt_qmatmul_group", a, m, (_lib.QWeight * count)(*structs), count, pointers(*outputs),
+              None if biases is None else pointers(*biases), accumulate, alpha, (stream or default_stream()).handle)
+
+
 class MatMul:
     """The quantized half of ``object MatMul``."""
 
@@ -122,12 +130,9 @@ class MatMul:
             nc = _nbytes(c)
             if nc is not None and nc < m * w.columns * 4:
                 raise _lib.IllegalArgumentException(f"output has {nc // 4} elements, needs {m} × {w.columns}")
-        structs = (_lib.QWeight * count)(*[w.qweight for w in weights])
-        outs = (ctypes.c_void_p * count)(*[_ptr(c) for c in outputs])
-        bias_arr = None if biases is None else (ctypes.c_void_p * count)(
-            *[None if b is None else _ptr(b) for b in biases])
-        _lib.call("kt_qmatmul_group", _ptr(a), int(m), structs, count, outs, bias_arr, int(bool(accumulate)),
-                  ctypes.c_float(alpha), (stream or default_stream()).handle)
+        _call_group(_ptr(a), int(m), [w.qweight for w in weights], [_ptr(c) for c in outputs],
+                    None if biases is None else [None if b is None else _ptr(b) for b in biases],
+                    int(bool(accumulate)), alpha, stream)
 
     @staticmethod
     def multiply_by_quantized_transposed(dy, weight: QuantizedTensor, dx, m: int, accumulate: bool = True,
