@@ -636,6 +636,188 @@ __global__ void __launch_bounds__(THREADS) attention_kernel(AttnArgs a) {
     }
 }
 
+// ---- decode attention of short contexts: one workgroup per query head ----------------------
+// Up to DIRECT_KEYS keys of 64 dims for one token: workgroup (kv head g, query head y of its
+// group), 16 waves, no key splits, so nothing meets in memory. Sixteen lanes hold a key row
+// (four dims each, as a coalesced load of four rows a wave leaves them), the score is their
+// DPP sum, and the sixteen keep their own running maximum, sum and weighted values: the loop
+// has no LDS access and no barrier. The query heads of a group read the same keys, on one
+// XCD (blockIdx.x is the kv head), from its L2.
+// Bound by the CU's read rate (512 bytes a key, 107 GB/s; two passes' loads in flight were no
+// faster) behind the launch and the first loads' latency. 32 query and 8 kv heads, traced:
+// 64 keys 5.5 us (with key splits 6.0), 200 5.6 (8.8), 400 6.7 (8.8), 544 7.9 (8.7), 800 9.2
+// (8.6); 14 and 2 heads 200 keys 5.6 (11.5), 800 9.0 (12.1).
+constexpr int DIRECT_KEYS = 640;
+constexpr int DIRECT_WAVES = 16;
+constexpr int DIRECT_QUADS = 4;  // key rows a lane holds at a time
+constexpr int DIRECT_PASS = DIRECT_WAVES * DIRECT_QUADS * 4;
+
+// Sum over the 16 lanes of a row, in every lane of it.
+__device__ __forceinline__ float row_sum_dpp(float v) {
+    v += dpp_move<0xB1>(v);
+    v += dpp_move<0x4E>(v);
+    v += dpp_move<0x141>(v);
+    return v + dpp_move<0x140>(v);
+}
+
+// This lane's four dims of a head of 64 rotated: lanes 0 .. 7 of a row hold dims 0 .. 31,
+// their pairs' other halves are eight lanes on.
+__device__ __forceinline__ f4 rope_row(f4 x, f4 c, f4 s, bool upper) {
+    f4 y;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float o = dpp_move<0x128>(x[e]);  // row_ror:8
+        float y1, y2;
+        rope_apply(upper ? o : x[e], upper ? x[e] : o, c[e], s[e], y1, y2);
+        y[e] = upper ? y2 : y1;
+    }
+    return y;
+}
+
+__global__ void __launch_bounds__(64 * DIRECT_WAVES) attention_direct_kernel(AttnArgs a) {
+    constexpr int HD = 64, HALF = 32;
+    __shared__ __attribute__((aligned(16))) float cs[2][HALF];
+    __shared__ __attribute__((aligned(16))) float part[DIRECT_WAVES][HD];
+    __shared__ float pm[DIRECT_WAVES], pl[DIRECT_WAVES];
+    const int32_t g = blockIdx.x, head = g * gridDim.y + blockIdx.y;
+    const int32_t tid = threadIdx.x, lane = tid & 63, c = lane & 15;
+    const int32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const size_t base = (static_cast<size_t>(a.layer) * a.num_kv_heads + g) * a.max_seq;  // row of key 0
+    const float* kbase = a.ck + base * HD + 4 * c;
+    const float* vbase = a.cv + base * HD + 4 * c;
+    const int32_t key0 = wave * (4 * DIRECT_QUADS) + (lane >> 4);  // this lane's first key of a pass
+
+    const f4 q0 = *reinterpret_cast<const f4*>(a.q + head * HD + 4 * c);
+    f4 kn = {0.0f, 0.0f, 0.0f, 0.0f}, vn = kn;
+    float ifr = 0.0f;
+    const bool cache_read = a.rope_cache && a.layer != 0;
+    uint32_t ce[4] = {0u, 0u, 0u, 0u};
+    if (a.rope) {
+        kn = load_any<f4>(a.k_new + g * HD + 4 * c);
+        vn = load_any<f4>(a.v_new + g * HD + 4 * c);
+        if (tid < HALF) {
+            ifr = a.inv_freq[tid];
+            if (cache_read) {
+#pragma unroll
+                for (int w = 0; w < 4; ++w)
+                    ce[w] = __hip_atomic_load(a.rope_cache + 4 * tid + w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            }
+        }
+    }
+    // the first pass's rows, whose addresses do not wait for the position
+    f4 k[DIRECT_QUADS], v[DIRECT_QUADS];
+    auto load = [&](f4 (&d)[DIRECT_QUADS], const float* rows, int32_t k0) {
+#pragma unroll
+        for (int u = 0; u < DIRECT_QUADS; ++u)
+            d[u] = *reinterpret_cast<const f4*>(rows + static_cast<size_t>(min(k0 + key0 + 4 * u, a.max_seq - 1)) * HD);
+    };
+    load(k, kbase, 0);
+    load(v, vbase, 0);
+    const int32_t pos = *a.position;
+    const int32_t n = min(pos + 1, a.max_seq);  // never read outside the cache
+    f4 q = q0;
+    if (a.rope) {
+        if (tid < HALF) {
+            float cf, sf;
+            if (cache_read && ce[0] == static_cast<uint32_t>(pos) + 1u && ce[1] == __builtin_bit_cast(uint32_t, ifr)) {
+                cf = __builtin_bit_cast(float, ce[2]);
+                sf = __builtin_bit_cast(float, ce[3]);
+            } else {
+                rope_cos_sin(pos, ifr, cf, sf);
+            }
+            cs[0][tid] = cf;
+            cs[1][tid] = sf;
+            if (a.rope_cache && a.layer == 0 && g == 0 && blockIdx.y == 0) {
+                uint32_t* e = a.rope_cache + 4 * tid;
+                __hip_atomic_store(e, static_cast<uint32_t>(pos) + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                __hip_atomic_store(e + 1, __builtin_bit_cast(uint32_t, ifr), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                __hip_atomic_store(e + 2, __builtin_bit_cast(uint32_t, cf), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                __hip_atomic_store(e + 3, __builtin_bit_cast(uint32_t, sf), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            }
+        }
+        __syncthreads();
+        const f4 cv4 = *reinterpret_cast<const f4*>(&cs[0][4 * (c & 7)]), sv4 = *reinterpret_cast<const f4*>(&cs[1][4 * (c & 7)]);
+        q = rope_row(q0, cv4, sv4, c >= 8);
+        kn = rope_row(kn, cv4, sv4, c >= 8);
+        if (tid < 16 && blockIdx.y == 0 && pos >= 0 && pos < a.max_seq) {  // the append, for later steps
+            *reinterpret_cast<f4*>(const_cast<float*>(kbase) + static_cast<size_t>(pos) * HD) = kn;
+            *reinterpret_cast<f4*>(const_cast<float*>(vbase) + static_cast<size_t>(pos) * HD) = vn;
+        }
+    }
+    const float qscale = a.scale * 1.4426950408889634f;  // scores in powers of two
+#pragma unroll
+    for (int e = 0; e < 4; ++e) q[e] *= qscale;
+
+    float m = -INFINITY, l = 0.0f;
+    f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int32_t k0 = 0; k0 < n; k0 += DIRECT_PASS) {
+        const bool more = k0 + DIRECT_PASS < n;  // the next pass's rows go out as registers become free
+        float p[DIRECT_QUADS], m_new = m;
+#pragma unroll
+        for (int u = 0; u < DIRECT_QUADS; ++u) {
+            const int32_t key = k0 + key0 + 4 * u;
+            if (a.rope && key == pos) {  // the new row, whatever the load saw
+                k[u] = kn;
+                v[u] = vn;
+            }
+            float d = k[u][0] * q[0];
+#pragma unroll
+            for (int e = 1; e < 4; ++e) d = fmaf(k[u][e], q[e], d);
+            d = row_sum_dpp(d);
+            p[u] = key < n ? d : -INFINITY;
+            m_new = fmaxf(m_new, p[u]);
+        }
+        if (more) load(k, kbase, k0 + DIRECT_PASS);
+        const float m_use = m_new == -INFINITY ? 0.0f : m_new;  // no key of these lanes yet
+        const float alpha = __builtin_amdgcn_exp2f(m - m_use);
+        m = m_new;
+        l *= alpha;
+        acc *= alpha;
+#pragma unroll
+        for (int u = 0; u < DIRECT_QUADS; ++u) {
+            p[u] = __builtin_amdgcn_exp2f(p[u] - m_use);
+            l += p[u];
+            const bool seen = k0 + key0 + 4 * u < n;  // (a row past the last key may hold anything)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] = fmaf(p[u], seen ? v[u][e] : 0.0f, acc[e]);
+        }
+        if (more) load(v, vbase, k0 + DIRECT_PASS);
+    }
+    // the four rows of a wave, then the waves in order
+    float mw = fmaxf(m, __shfl_xor(m, 16));
+    mw = fmaxf(mw, __shfl_xor(mw, 32));
+    const float w = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mw);
+    l *= w;
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        acc[e] *= w;
+        acc[e] += __shfl_xor(acc[e], 16);
+        acc[e] += __shfl_xor(acc[e], 32);
+    }
+    if (lane < 16) *reinterpret_cast<f4*>(&part[wave][4 * c]) = acc;
+    if (lane == 0) {
+        pm[wave] = mw;
+        pl[wave] = l;
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    const float mi = pm[c];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < DIRECT_WAVES; ++i) mx = fmaxf(mx, lane_value(mi, i));
+    const float wi = mi == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mi - mx);
+    const float li = pl[c] * wi;
+    float x = 0.0f, sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < DIRECT_WAVES; ++i) {
+        x = fmaf(part[i][lane], lane_value(wi, i), x);
+        sum += lane_value(li, i);
+    }
+    a.context[head * HD + lane] = x * (1.0f / sum);
+}
+
 // ---- prefill attention: blocked over queries, fp32 precision on the bf16 matrix units -----
 // Workgroup (kv head g, block of 64 / G consecutive tokens): the query rows
 // r = (token t0 + r / G, head g G + r % G), r < 64, over keys 0 .. position + token, 64 keys
@@ -1161,6 +1343,35 @@ static int32_t attention_launch(const float* q, int32_t tokens, const int32_t* p
                                                                                           paired);
         }
         KT_LAUNCHED("prefill attention kernel");
+        return KT_OK;
+    }
+    if (tokens == 1 && head_dim == 64 && key_bound <= DIRECT_KEYS) {
+        // one token over a short context: a workgroup per query head
+        AttnArgs a{};
+        a.q = q;
+        a.position = position;
+        a.ck = cache_k;
+        a.cv = cache_v;
+        a.context = context;
+        a.layer = layer;
+        a.max_seq = max_seq;
+        a.num_heads = num_heads;
+        a.num_kv_heads = num_kv_heads;
+        a.head_dim = head_dim;
+        a.scale = 1.0f / sqrtf(static_cast<float>(head_dim));
+        a.k_new = k_new;
+        a.v_new = v_new;
+        a.inv_freq = inv_freq;
+        a.rope = k_new != nullptr ? 1 : 0;
+        if (a.rope && workspace_fits(st, 0)) {  // (without one the launch computes cos and sin itself)
+            uint32_t* counters = nullptr;
+            void* general = nullptr;
+            const int32_t status = workspace_counters(st, 0, 0, &general, &counters);
+            if (status) return status;
+            a.rope_cache = counters + ROPE_CACHE_WORD;
+        }
+        attention_direct_kernel<<<dim3(static_cast<uint32_t>(num_kv_heads), static_cast<uint32_t>(G)), 64 * DIRECT_WAVES, 0, st>>>(a);
+        KT_LAUNCHED("attention kernel");
         return KT_OK;
     }
     // Key splits: enough workgroups to fill the GPU when few tokens attend.

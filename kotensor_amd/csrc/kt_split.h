@@ -10,6 +10,14 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+// 16 bytes at any alignment (dword accesses need none in global memory).
+template <typename T>
+__device__ __forceinline__ T load_any(const void* p) {
+    T v;
+    __builtin_memcpy(&v, p, sizeof(T));
+    return v;
+}
+
 // The upper halves of two floats in one dword: their bf16 truncations.
 __device__ __forceinline__ uint32_t upper_halves(float lo, float hi) {
     return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, hi), __builtin_bit_cast(uint32_t, lo), 0x07060302u);

@@ -30,14 +30,6 @@ constexpr int STEP = 64;          // elements of the summed dimension per step
 constexpr int PITCH = STEP + 8;   // halfs per LDS row: 16-byte reads of 16 consecutive rows hit all banks once
 constexpr int MAX_SPLITS = 32;
 
-// 16 bytes at any alignment (dword accesses need none in global memory).
-template <typename T>
-__device__ __forceinline__ T load_any(const void* p) {
-    T v;
-    __builtin_memcpy(&v, p, sizeof(T));
-    return v;
-}
-
 // The dword at byte i of a row of `bytes` >= 4 bytes; bytes past the row's end are any.
 __device__ __forceinline__ uint32_t load_end(const void* row, int32_t i, int32_t bytes) {
     const int32_t at = min(i, bytes - 4);

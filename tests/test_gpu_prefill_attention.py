@@ -1,6 +1,6 @@
-"""The prefill attention (kt_decoder.hip, fp32 precision by products of bf16 parts) against
-64 bits: blocks of 64 query rows that end inside a token's heads, tiles of 64 keys with
-every kind of end, a wave without keys of its own, both orders of the blocks, both head
+"""The prefill attention and the one-token attention of short contexts (kt_decoder.hip)
+against 64 bits. Prefill: blocks of query rows that end inside a token's heads, key tiles
+with every kind of end, a wave without keys of its own, both orders of the blocks, both head
 dimensions; and rows with infinities.
 
 Bound: six products of parts per element leave an fp32 rounding each; with the fp32 sums of
@@ -51,6 +51,19 @@ def test_prefill_attention_against_64_bits(kt, tokens, start, heads, kvh, d):
     keys[:, start + tokens:] = np.nan  # past the last key: never used
     err = normwise_rel(_call(kt, q, keys, values, start, heads), _exact(q, keys, values, start, heads))
     print(f"  error {err:.2e}", flush=True)
+    assert err <= 1e-6
+
+
+@pytest.mark.parametrize("start,heads,kvh", [(0, 32, 8), (15, 14, 2), (16, 1, 1), (255, 8, 8), (256, 32, 8), (511, 9, 1), (639, 16, 2)])
+def test_one_token_of_a_short_context_against_64_bits(kt, start, heads, kvh):
+    """The kernel of one workgroup per query head: a wave's rows, passes of 256 keys and the
+    longest context it takes; also inside a longer cache than its keys."""
+    banner("one-token-attention", start, heads, kvh)
+    rng = np.random.default_rng(start)
+    q = (2.0 * rng.standard_normal((1, heads * 64))).astype(np.float32)
+    keys, values = (rng.standard_normal((kvh, start + 40, 64)).astype(np.float32) for _ in range(2))
+    keys[:, start + 1:], values[:, start + 1:] = np.nan, np.nan  # never used
+    err = normwise_rel(_call(kt, q, keys, values, start, heads), _exact(q, keys, values, start, heads))
     assert err <= 1e-6
 
 
