@@ -1102,6 +1102,247 @@ __global__ void __launch_bounds__(THREADS, HD == 64 ? 2 : 1)
     }
 }
 
+// ---- prefill attention on keys and values split beforehand ---------------------------------
+// The same products with K and V split once for all query rows: prefill_parts_kernel writes
+// their parts to the workspace in the order of the matrix products' lanes, so that a wave
+// loads an operand as one contiguous KiB and the main loop has neither LDS nor barriers.
+// Workgroup (kv head g, block of 32 / G consecutive tokens): 32 query rows; wave w takes the
+// 32-key blocks w, w + 4, ...; the four waves' sums meet through LDS at the end.
+// Per query row the tile kernel above also splits every key and value; here a wave and block
+// has about 345 vector instructions beside its 48 matrix products, and 24 KiB of operands
+// from L2. Traced (tile kernel -> this with its 5 us of splitting): 1024 tokens, 32 query and
+// 8 kv heads of 64 48 -> 42 us; with the call 512 tokens 25 -> 19, 64 after 1024 44 -> 21, 17
+// after 900 40 -> 19; heads of 128 1024 tokens 118 -> 84. Short contexts stay with the tile
+// kernel's one launch (100 tokens, 14 heads: 9.6 against 15 us; 200 of 128 dims 26 against 18),
+// so do calls whose parts have no workspace.
+constexpr int SPLIT_ROWS = 32;
+constexpr int PARTS_MIN_KEYS = 192;
+constexpr size_t MAX_PARTS_BYTES = 64 << 20;  // longer caches: the kernel that splits tiles itself
+
+// Parts of one 32-key block of a kv head: K [HD / 16][3] and V [2][HD / 32][3] operands of
+// 1 KiB (64 lanes of 16 bytes).
+__host__ __device__ constexpr size_t parts_block_bytes(int hd) { return static_cast<size_t>(hd / 16 * 3 + 2 * (hd / 32) * 3) * 1024; }
+
+// Workgroup (kv head, 64-key tile): groups of eight values as attention_prefill_kernel stages
+// them. Keys past the last one repeat it.
+template <int HD>
+__global__ void __launch_bounds__(THREADS) prefill_parts_kernel(AttnArgs a, int32_t tokens, int32_t blocks, uint8_t* parts) {
+    const int32_t g = blockIdx.x, k0 = blockIdx.y * PKT;
+    const int32_t n_keys = min(*a.position + tokens, a.max_seq);
+    if (k0 >= n_keys) return;
+    const size_t base = (static_cast<size_t>(a.layer) * a.num_kv_heads + g) * a.max_seq;
+    uint8_t* out = parts + (static_cast<size_t>(g) * blocks + k0 / 32) * parts_block_bytes(HD);
+#pragma unroll
+    for (int i = 0; i < PKT * HD / 8 / THREADS; ++i) {
+        const int32_t e = threadIdx.x + i * THREADS;
+        float v[8];
+        bf16x8 part[3];
+        const int32_t key = e / (HD / 8), o = e % (HD / 8);  // K: dims 8 o .. + 7 of a key
+        const f4* src = reinterpret_cast<const f4*>(a.ck + (base + min(k0 + key, n_keys - 1)) * HD + 8 * o);
+        const f4 v0 = src[0], v1 = src[1];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            v[u] = v0[u];
+            v[4 + u] = v1[u];
+        }
+        split3(v, part);
+        uint8_t* ko = out + (key >> 5) * parts_block_bytes(HD) + (o >> 1) * 3072 + ((key & 31) + 32 * (o & 1)) * 16;
+#pragma unroll
+        for (int h = 0; h < 3; ++h) *reinterpret_cast<bf16x8*>(ko + h * 1024) = part[h];
+        const int32_t d = e % HD, oct = e / HD;  // V: dim d of keys 16 (oct / 2) + 4 (oct % 2) + {0 .. 3, 8 .. 11}
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            v[u] = a.cv[(base + min(k0 + 16 * (oct >> 1) + 4 * (oct & 1) + (u & 3) + 8 * (u >> 2), n_keys - 1)) * HD + d];
+        split3(v, part);
+        uint8_t* vo = out + (oct >> 2) * parts_block_bytes(HD) + HD / 16 * 3072 +
+                      (((oct >> 1) & 1) * (HD / 32) + (d >> 5)) * 3072 + ((d & 31) + 32 * (oct & 1)) * 16;
+#pragma unroll
+        for (int h = 0; h < 3; ++h) *reinterpret_cast<bf16x8*>(vo + h * 1024) = part[h];
+    }
+}
+
+template <int HD>
+__global__ void __launch_bounds__(THREADS, HD == 64 ? 2 : 1)
+    attention_parts_kernel(AttnArgs a, int32_t tokens, int32_t qb_tokens, int32_t nqb, int32_t blocks, const uint8_t* parts) {
+    constexpr int DB = HD / 32, QS = HD / 16;
+    __shared__ float ex[THREADS / 64 - 1][DB * 16 + 2][64];
+    const int32_t g = blockIdx.x, qb = nqb - 1 - static_cast<int32_t>(blockIdx.y);
+    const int32_t G = a.num_heads / a.num_kv_heads;
+    const int32_t dim = a.num_heads * HD;
+    const int32_t t0 = qb * qb_tokens, t_end = min(t0 + qb_tokens, tokens);
+    const int32_t P0 = *a.position;
+    const int32_t n_keys = min(P0 + t_end, a.max_seq);
+    const int32_t tid = threadIdx.x, lane = tid & 63, hl = lane >> 5, r = lane & 31;
+    const int32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+    const int32_t tl = r / G, tok = t0 + tl;
+    const bool row_ok = tl < qb_tokens && tok < t_end;
+    const int32_t head = g * G + r % G;
+    const int32_t p_r = row_ok ? min(P0 + tok, a.max_seq - 1) : -1;  // last key of the row
+    const int32_t p_min = min(P0 + t0, a.max_seq - 1);               // of the block's first token
+    const size_t qat = static_cast<size_t>(min(tok, tokens - 1)) * dim + head * HD;
+
+    bf16x8 qp[QS][3];  // as attention_prefill_kernel's
+    const float qscale = a.scale * 1.4426950408889634f;
+#pragma unroll
+    for (int s = 0; s < QS; ++s) {
+        const f4* src = reinterpret_cast<const f4*>(a.q + qat + 16 * s + 8 * hl);
+        const f4 v0 = src[0], v1 = src[1];
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[e] = v0[e] * qscale;
+            v[4 + e] = v1[e] * qscale;
+        }
+        split3(v, qp[s]);
+    }
+
+    const int32_t n_blocks = min((n_keys + 31) / 32, blocks);
+    const uint8_t* base = parts + static_cast<size_t>(g) * blocks * parts_block_bytes(HD) + lane * 16;
+    auto operand = [&](int32_t kb, int i) {  // operand i of block kb
+        return *reinterpret_cast<const bf16x8*>(base + static_cast<size_t>(kb) * parts_block_bytes(HD) + i * 1024);
+    };
+    f32x16 oacc[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) oacc[db][e] = 0.0f;
+    float m = -INFINITY, l = 0.0f;
+    bf16x8 kp[QS][3];
+    if (wave < n_blocks) {
+#pragma unroll
+        for (int i = 0; i < 3 * QS; ++i) kp[i / 3][i % 3] = operand(wave, i);
+    }
+    for (int32_t kb = wave; kb < n_blocks; kb += THREADS / 64) {
+        bf16x8 vp[2][DB][3];  // the values' loads go out before the scores are made
+#pragma unroll
+        for (int i = 0; i < 6 * DB; ++i) vp[i / (3 * DB)][i / 3 % DB][i % 3] = operand(kb, 3 * QS + i);
+        __builtin_amdgcn_sched_barrier(0);
+        f32x16 big, small;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) big[e] = small[e] = 0.0f;
+#pragma unroll
+        for (int s = 0; s < QS; ++s) {
+            small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kp[s][2], qp[s][0], small, 0, 0, 0);
+            small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kp[s][0], qp[s][2], small, 0, 0, 0);
+            small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kp[s][1], qp[s][1], small, 0, 0, 0);
+            small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kp[s][1], qp[s][0], small, 0, 0, 0);
+            small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kp[s][0], qp[s][1], small, 0, 0, 0);
+            big = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kp[s][0], qp[s][0], big, 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const int32_t nk = min(kb + THREADS / 64, n_blocks - 1);  // the wave's next block's keys
+#pragma unroll
+        for (int i = 0; i < 3 * QS; ++i) kp[i / 3][i % 3] = operand(nk, i);
+        __builtin_amdgcn_sched_barrier(0);
+        const int32_t k0 = 32 * kb;
+        float p[16], tmax = -INFINITY;
+        const bool masked = k0 + 31 > p_min;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            p[e] = big[e] + small[e];
+            if (masked) p[e] = k0 + 8 * (e >> 2) + 4 * hl + (e & 3) <= p_r ? p[e] : -INFINITY;
+            tmax = fmaxf(tmax, p[e]);
+        }
+        tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+        const float m_new = fmaxf(m, tmax);
+        const float m_use = m_new == -INFINITY ? 0.0f : m_new;  // no key of the row yet
+        const float alpha = __builtin_amdgcn_exp2f(m - m_use);
+        float psum = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            p[e] = __builtin_amdgcn_exp2f(p[e] - m_use);
+            psum += p[e];
+        }
+        l = l * alpha + psum;
+        m = m_new;
+        bf16x8 pp[2][3];
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = p[8 * st + e];
+            split3(v, pp[st]);
+        }
+#pragma unroll
+        for (int db = 0; db < DB; ++db) {
+            f32x16 sum;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) sum[e] = 0.0f;
+#pragma unroll
+            for (int st = 0; st < 2; ++st) {
+                sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vp[st][db][2], pp[st][0], sum, 0, 0, 0);
+                sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vp[st][db][0], pp[st][2], sum, 0, 0, 0);
+                sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vp[st][db][1], pp[st][1], sum, 0, 0, 0);
+                sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vp[st][db][1], pp[st][0], sum, 0, 0, 0);
+                sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vp[st][db][0], pp[st][1], sum, 0, 0, 0);
+            }
+#pragma unroll
+            for (int st = 0; st < 2; ++st)
+                sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vp[st][db][0], pp[st][0], sum, 0, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 16; ++e) oacc[db][e] = fmaf(oacc[db][e], alpha, sum[e]);
+        }
+    }
+    l += __shfl_xor(l, 32);
+    if (wave != 0) {
+#pragma unroll
+        for (int i = 0; i < DB * 16; ++i) ex[wave - 1][i][lane] = oacc[i / 16][i % 16];
+        ex[wave - 1][DB * 16][lane] = m;
+        ex[wave - 1][DB * 16 + 1][lane] = l;
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    float ms[4] = {m, ex[0][DB * 16][lane], ex[1][DB * 16][lane], ex[2][DB * 16][lane]};
+    const float mx = fmaxf(fmaxf(ms[0], ms[1]), fmaxf(ms[2], ms[3]));
+    const float m_use = mx == -INFINITY ? 0.0f : mx;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ms[i] = __builtin_amdgcn_exp2f(ms[i] - m_use);
+    float sum = l * ms[0];
+#pragma unroll
+    for (int i = 1; i < 4; ++i) sum = fmaf(ex[i - 1][DB * 16 + 1][lane], ms[i], sum);
+    const float inv = 1.0f / sum;
+    float* dst = a.context + qat;
+    bool nan = false;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            f4 o;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float x = oacc[db][4 * c + i] * ms[0];
+#pragma unroll
+                for (int w = 1; w < 4; ++w) x = fmaf(ex[w - 1][db * 16 + 4 * c + i][lane], ms[w], x);
+                o[i] = x * inv;
+                nan = nan || o[i] != o[i];
+            }
+            if (row_ok) *reinterpret_cast<f4*>(dst + db * 32 + 8 * c + 4 * hl) = o;
+        }
+    uint64_t rows = __ballot(nan && row_ok);
+    rows = (rows | rows >> 32) & 0xFFFFFFFFull;
+    const size_t kv_base = (static_cast<size_t>(a.layer) * a.num_kv_heads + g) * a.max_seq;
+    while (rows) {
+        const int32_t rr = __builtin_ctzll(rows), tt = t0 + rr / G, hh = g * G + rr % G;
+        rows &= rows - 1;
+        const size_t at = static_cast<size_t>(tt) * dim + hh * HD;
+        attend_row<HD>(a, a.q + at, kv_base, min(P0 + tt, a.max_seq - 1) + 1, a.context + at, &ex[0][0][0]);
+    }
+}
+
+template <int HD>
+int32_t launch_prefill_parts(const AttnArgs& a, int32_t tokens, int32_t key_bound, uint8_t* parts, hipStream_t st) {
+    const int32_t blocks = 2 * ceil_div(key_bound, PKT);  // whole tiles
+    const int32_t G = a.num_heads / a.num_kv_heads, qb_tokens = SPLIT_ROWS / G, nqb = ceil_div(tokens, qb_tokens);
+    prefill_parts_kernel<HD><<<dim3(static_cast<uint32_t>(a.num_kv_heads), static_cast<uint32_t>(blocks / 2)), THREADS, 0, st>>>(
+        a, tokens, blocks, parts);
+    KT_LAUNCHED("prefill attention: parts");
+    attention_parts_kernel<HD><<<dim3(static_cast<uint32_t>(a.num_kv_heads), static_cast<uint32_t>(nqb)), THREADS, 0, st>>>(
+        a, tokens, qb_tokens, nqb, blocks, parts);
+    KT_LAUNCHED("prefill attention kernel");
+    return KT_OK;
+}
+
 // ---- SwiGLU gate -----------------------------------------------------------------------
 __global__ void __launch_bounds__(THREADS) silu_mul_kernel(float* __restrict__ gate, const float* __restrict__ up,
                                                            int64_t n) {
@@ -1326,6 +1567,15 @@ static int32_t attention_launch(const float* q, int32_t tokens, const int32_t* p
         a.head_dim = head_dim;
         a.scale = 1.0f / sqrtf(static_cast<float>(head_dim));
         a.splits = 1;
+        const size_t parts_bytes = static_cast<size_t>(num_kv_heads) * 2 * ceil_div(key_bound, PKT) *
+                                   (head_dim == 64 ? parts_block_bytes(64) : parts_block_bytes(128));
+        if (key_bound >= PARTS_MIN_KEYS && G <= SPLIT_ROWS && parts_bytes <= MAX_PARTS_BYTES && workspace_fits(st, parts_bytes)) {
+            void* parts = nullptr;
+            const int32_t status = workspace(st, parts_bytes, &parts);
+            if (status) return status;
+            return head_dim == 64 ? launch_prefill_parts<64>(a, tokens, key_bound, static_cast<uint8_t*>(parts), st)
+                                  : launch_prefill_parts<128>(a, tokens, key_bound, static_cast<uint8_t*>(parts), st);
+        }
         const int32_t qb_tokens = PQ_ROWS / G;
         const int32_t nqb = ceil_div(tokens, qb_tokens);
         const dim3 grid(static_cast<uint32_t>(num_kv_heads), static_cast<uint32_t>(nqb));

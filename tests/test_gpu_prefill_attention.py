@@ -41,6 +41,7 @@ def _exact(q, keys, values, start, heads):
 @pytest.mark.parametrize("tokens,start,heads,kvh,d", [
     (16, 0, 4, 4, 64), (17, 47, 14, 2, 64), (64, 0, 32, 8, 64), (65, 63, 8, 1, 64), (100, 1500, 4, 1, 64),
     (700, 1, 8, 8, 64), (16, 0, 8, 8, 128), (33, 95, 16, 2, 128), (130, 200, 7, 1, 128), (40, 3, 3, 1, 64),
+    (191, 0, 8, 8, 64), (160, 32, 14, 2, 64), (33, 190, 8, 1, 128), (16, 240, 9, 1, 64), (257, 0, 5, 5, 128),
 ])
 def test_prefill_attention_against_64_bits(kt, tokens, start, heads, kvh, d):
     banner("prefill-attention", tokens, start, heads, kvh, d)
@@ -52,6 +53,41 @@ def test_prefill_attention_against_64_bits(kt, tokens, start, heads, kvh, d):
     err = normwise_rel(_call(kt, q, keys, values, start, heads), _exact(q, keys, values, start, heads))
     print(f"  error {err:.2e}", flush=True)
     assert err <= 1e-6
+
+
+def test_prefill_attention_recorded_without_workspace(kt):
+    """Recorded on a stream that never ran eagerly there is no workspace for the parts: the
+    kernel that splits tiles itself runs; its replays equal the 64-bit result, with eager
+    calls (on parts) in between."""
+    import ctypes
+
+    from kotensor_amd import _lib
+    tokens, heads, kvh, d = 210, 8, 2, 64
+    rng = np.random.default_rng(3)
+    q = rng.standard_normal((tokens, heads * d)).astype(np.float32)
+    keys, values = (rng.standard_normal((kvh, tokens, d)).astype(np.float32) for _ in range(2))
+    want = _exact(q, keys, values, 0, heads)
+    dq, dk, dv, pos = (kt.DeviceBuffer.from_numpy(a) for a in (q, keys, values, np.zeros(1, np.int32)))
+    out, stream, graph = kt.DeviceBuffer(q.nbytes), kt.Stream.create(), ctypes.c_void_p()
+    kt.synchronize()
+    banner("prefill-attention-record")
+    _lib.call("kt_graph_begin", stream.handle)
+    try:
+        _lib.call("kt_attention", dq.ptr, tokens, pos.ptr, tokens, dk.ptr, dv.ptr, 0, tokens, heads, kvh, d, out.ptr, stream.handle)
+    finally:
+        _lib.call("kt_graph_end", stream.handle, ctypes.byref(graph))
+    try:
+        for _ in range(3):
+            out.fill_zero()
+            kt.synchronize()
+            _lib.call("kt_graph_launch", graph, stream.handle)
+            stream.synchronize()
+            assert normwise_rel(out.download(np.float32).reshape(q.shape), want) <= 1e-6
+            assert normwise_rel(_call(kt, q, keys, values, 0, heads), want) <= 1e-6
+    finally:
+        stream.synchronize()
+        _lib.call("kt_graph_destroy", graph)
+        stream.destroy()
 
 
 @pytest.mark.parametrize("start,heads,kvh", [(0, 32, 8), (15, 14, 2), (16, 1, 1), (255, 8, 8), (256, 32, 8), (511, 9, 1), (639, 16, 2)])
@@ -67,11 +103,11 @@ def test_one_token_of_a_short_context_against_64_bits(kt, start, heads, kvh):
     assert err <= 1e-6
 
 
-@pytest.mark.parametrize("d", [64, 128])
-def test_prefill_attention_infinities(kt, d):
+@pytest.mark.parametrize("d,tokens", [(64, 70), (128, 70), (64, 200), (128, 200)])
+def test_prefill_attention_infinities(kt, d, tokens):
     """A key whose score is minus infinity adds nothing, an infinite value makes infinities
     of the rows that see it, a NaN query NaNs of its own row; other rows keep their values."""
-    tokens, heads, kvh = 70, 4, 2
+    heads, kvh = 4, 2
     rng = np.random.default_rng(7)
     q = rng.standard_normal((tokens, heads * d)).astype(np.float32)
     q[:, ::d] = np.abs(q[:, ::d]) + 0.1  # each head's first dim positive
@@ -81,7 +117,7 @@ def test_prefill_attention_infinities(kt, d):
     keys[0, 5, 0] = -np.inf
     values[1, 60, 3] = np.inf
     q[20, 2 * d + 1] = np.nan
-    banner("prefill-attention-inf", d)
+    banner("prefill-attention-inf", d, tokens)
     got = _call(kt, q, keys, values, 0, heads)
     plain = keys.copy()
     plain[0, 5, 0] = -1e6  # the same weights: nothing
