@@ -66,6 +66,13 @@ WaitLimits wait_limits();
 // way to do without.
 bool workspace_fits(hipStream_t stream, size_t bytes);
 
+// The stream's area for the fused loss (kept for its next call, freed with the stream), or
+// nullptr: beyond LOSS_AREA_BYTES, while the stream is captured (a graph outlives calls), or
+// while another thread's call has it. A call that got it says when its work is enqueued.
+constexpr size_t LOSS_AREA_BYTES = size_t(192) << 20;
+int32_t loss_area(hipStream_t stream, size_t bytes, void** out);
+void loss_area_done(hipStream_t stream);
+
 // Validated view of a kt_qweight, with the derived layout numbers.
 struct WeightView {
     const uint8_t* q;

@@ -36,10 +36,13 @@ struct Block {
     size_t bytes = 0;       // whole allocation
     size_t zbytes = 0;      // the zeroed accumulator region after the counters
     bool captured = false;  // handed to a kernel recorded into a graph
+    bool busy = false;      // a loss area handed to a call that is still enqueuing
     int32_t fault = -1;     // the stream's slot of the fault words, once a kernel took it
 };
 std::mutex g_ws_mutex;
 std::map<std::pair<int, hipStream_t>, Block> g_ws;
+// The fused loss's areas, beside the workspaces its products use (loss_area).
+std::map<std::pair<int, hipStream_t>, Block> g_loss;
 // Blocks replaced or orphaned while a recorded graph may still address them. A graph
 // keeps the addresses it was recorded with, and graphs can outlive their stream, so
 // these stay allocated until the process ends (each is smaller than its successor, so
@@ -144,6 +147,40 @@ bool workspace_fits(hipStream_t stream, size_t bytes) {
     std::lock_guard<std::mutex> lock(g_ws_mutex);
     const auto it = g_ws.find(std::make_pair(device, stream));
     return it != g_ws.end() && it->second.ptr && COUNTER_BYTES + it->second.zbytes + bytes <= it->second.bytes;
+}
+
+int32_t loss_area(hipStream_t stream, size_t bytes, void** out) {
+    *out = nullptr;
+    if (bytes > LOSS_AREA_BYTES) return KT_OK;
+    int device = 0;
+    KT_HIP(hipGetDevice(&device));
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    KT_HIP(hipStreamIsCapturing(stream, &capture));
+    if (capture != hipStreamCaptureStatusNone) return KT_OK;
+    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    Block& b = g_loss[std::make_pair(device, stream)];
+    if (b.busy) return KT_OK;  // another thread is enqueuing with it
+    if (b.bytes < bytes) {
+        if (b.ptr) {
+            KT_HIP(hipStreamSynchronize(stream));
+            KT_HIP(hipFree(b.ptr));
+            b = Block{};
+        }
+        const size_t want = bytes + bytes / 4 < LOSS_AREA_BYTES ? bytes + bytes / 4 : LOSS_AREA_BYTES;
+        KT_HIP(hipMalloc(&b.ptr, want));
+        b.bytes = want;
+    }
+    b.busy = true;
+    *out = b.ptr;
+    return KT_OK;
+}
+
+void loss_area_done(hipStream_t stream) {
+    int device = 0;
+    if (hipGetDevice(&device) != hipSuccess) return;
+    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    const auto it = g_loss.find(std::make_pair(device, stream));
+    if (it != g_loss.end()) it->second.busy = false;
 }
 
 int32_t workspace_counters(hipStream_t stream, size_t bytes, size_t count, void** general, uint32_t** counters) {
@@ -469,6 +506,11 @@ int32_t kt_stream_destroy(void* stream) {
             if (it->second.ptr && it->second.captured) g_retired.push_back(it->second.ptr);
             else if (it->second.ptr) KT_HIP(hipFree(it->second.ptr));
             g_ws.erase(it);
+        }
+        const auto loss = g_loss.find(std::make_pair(device, s));
+        if (loss != g_loss.end()) {
+            if (loss->second.ptr) KT_HIP(hipFree(loss->second.ptr));
+            g_loss.erase(loss);
         }
     }
     KT_HIP(hipStreamDestroy(s));

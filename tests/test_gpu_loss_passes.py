@@ -31,3 +31,23 @@ def test_passes_match_the_oracle(kt, oracle_lib, k, n, rows, bits, g):
     assert normwise_rel(bg, want_bg) <= TOL
     loss2, hg2, bg2 = _run(kt, head, hidden, targets)
     assert loss2 == loss and same_bits(hg, hg2) and same_bits(bg, bg2)
+
+
+def test_scratch_kept_with_the_stream(kt, oracle_lib):
+    """The scratch area grows and is reused between calls of different sizes on a stream, and
+    a stream made after another was destroyed starts without it: always the same bits."""
+    banner("fused-ce-scratch")
+    q, head, bias, hidden, targets = _setup(kt, oracle_lib, 64, 2000, 40, 4, 64, 3)
+    small = _run(kt, head, hidden[:3], targets[:3])
+    whole = _run(kt, head, hidden, targets)
+    for _ in range(2):
+        stream = kt.Stream.create()
+        for rows, want in ((3, small), (40, whole), (3, small)):
+            h = kt.DeviceTensor.from_numpy(hidden[:rows])
+            hg, bg = kt.DeviceTensor.zeros(h.shape), kt.DeviceTensor.zeros((1, head.out_size))
+            kt.synchronize()  # the zeros, on the null stream
+            out = kt.fused_cross_entropy_loss(h, head, targets[:rows], hidden_grad=hg, bias_grad=bg, stream=stream)
+            stream.synchronize()
+            assert out.item() == want[0]
+            assert same_bits(out.hidden_grad.numpy(), want[1]) and same_bits(out.bias_grad.numpy().reshape(-1), want[2])
+        stream.destroy()
