@@ -61,17 +61,23 @@ struct WaitLimits {
 };
 WaitLimits wait_limits();
 
-// Whether the stream's workspace can hold `bytes` of general area now (while it is being
-// captured it cannot grow; a caller's fixed workspace never does), for calls that have a
-// way to do without.
-bool workspace_fits(hipStream_t stream, size_t bytes);
+// Whether the stream has a workspace or may get one now (while it is being captured it may
+// not), for calls that have a way to do without its counter region.
+bool workspace_present(hipStream_t stream);
 
-// The stream's area for the fused loss (kept for its next call, freed with the stream), or
-// nullptr: beyond LOSS_AREA_BYTES, while the stream is captured (a graph outlives calls), or
-// while another thread's call has it. A call that got it says when its work is enqueued.
-constexpr size_t LOSS_AREA_BYTES = size_t(192) << 20;
-int32_t loss_area(hipStream_t stream, size_t bytes, void** out);
-void loss_area_done(hipStream_t stream);
+// An area of the stream that one call holds while it enqueues its launches (two threads on
+// one stream then never interleave launches on it), kept for the next call and freed with the
+// stream; nullptr where the call does without: more than `limit` bytes, another thread's call
+// in progress, a captured stream whose area is too small. (Calls on a caller's fixed
+// workspace get its general area.) The
+// split products' slices and the prefill attention's parts are CALL_SLICES; the fused loss's
+// scratch is CALL_LOSS, since its products want the other. A call that got one returns it
+// with call_area_done once its last launch is enqueued.
+enum CallArea { CALL_SLICES, CALL_LOSS, CALL_AREAS };
+int32_t call_area(CallArea kind, hipStream_t stream, size_t bytes, size_t limit, void** out);
+void call_area_done(CallArea kind, hipStream_t stream);
+constexpr size_t SLICES_LIMIT = size_t(64) << 20;
+constexpr size_t LOSS_LIMIT = size_t(192) << 20;
 
 // Validated view of a kt_qweight, with the derived layout numbers.
 struct WeightView {

@@ -1104,7 +1104,7 @@ __global__ void __launch_bounds__(THREADS, HD == 64 ? 2 : 1)
 
 // ---- prefill attention on keys and values split beforehand ---------------------------------
 // The same products with K and V split once for all query rows: prefill_parts_kernel writes
-// their parts to the workspace in the order of the matrix products' lanes, so that a wave
+// their parts to memory in the order of the matrix products' lanes, so that a wave
 // loads an operand as one contiguous KiB and the main loop has neither LDS nor barriers.
 // Workgroup (kv head g, block of 32 / G consecutive tokens): 32 query rows; wave w takes the
 // 32-key blocks w, w + 4, ...; the four waves' sums meet through LDS at the end.
@@ -1114,10 +1114,10 @@ __global__ void __launch_bounds__(THREADS, HD == 64 ? 2 : 1)
 // 8 kv heads of 64 48 -> 42 us; with the call 512 tokens 25 -> 19, 64 after 1024 44 -> 21, 17
 // after 900 40 -> 19; heads of 128 1024 tokens 118 -> 84. Short contexts stay with the tile
 // kernel's one launch (100 tokens, 14 heads: 9.6 against 15 us; 200 of 128 dims 26 against 18),
-// so do calls whose parts have no workspace.
+// so do calls that get no area for their parts (more than SLICES_LIMIT, a first call under
+// capture, another thread's call in progress).
 constexpr int SPLIT_ROWS = 32;
 constexpr int PARTS_MIN_KEYS = 192;
-constexpr size_t MAX_PARTS_BYTES = 64 << 20;  // longer caches: the kernel that splits tiles itself
 
 // Parts of one 32-key block of a kv head: K [HD / 16][3] and V [2][HD / 32][3] operands of
 // 1 KiB (64 lanes of 16 bytes).
@@ -1569,12 +1569,15 @@ static int32_t attention_launch(const float* q, int32_t tokens, const int32_t* p
         a.splits = 1;
         const size_t parts_bytes = static_cast<size_t>(num_kv_heads) * 2 * ceil_div(key_bound, PKT) *
                                    (head_dim == 64 ? parts_block_bytes(64) : parts_block_bytes(128));
-        if (key_bound >= PARTS_MIN_KEYS && G <= SPLIT_ROWS && parts_bytes <= MAX_PARTS_BYTES && workspace_fits(st, parts_bytes)) {
+        if (key_bound >= PARTS_MIN_KEYS && G <= SPLIT_ROWS) {
             void* parts = nullptr;
-            const int32_t status = workspace(st, parts_bytes, &parts);
-            if (status) return status;
-            return head_dim == 64 ? launch_prefill_parts<64>(a, tokens, key_bound, static_cast<uint8_t*>(parts), st)
-                                  : launch_prefill_parts<128>(a, tokens, key_bound, static_cast<uint8_t*>(parts), st);
+            if (const int32_t status = call_area(CALL_SLICES, st, parts_bytes, SLICES_LIMIT, &parts)) return status;
+            if (parts) {
+                const int32_t status = head_dim == 64 ? launch_prefill_parts<64>(a, tokens, key_bound, static_cast<uint8_t*>(parts), st)
+                                                      : launch_prefill_parts<128>(a, tokens, key_bound, static_cast<uint8_t*>(parts), st);
+                call_area_done(CALL_SLICES, st);
+                return status;
+            }
         }
         const int32_t qb_tokens = PQ_ROWS / G;
         const int32_t nqb = ceil_div(tokens, qb_tokens);
@@ -1613,7 +1616,7 @@ static int32_t attention_launch(const float* q, int32_t tokens, const int32_t* p
         a.v_new = v_new;
         a.inv_freq = inv_freq;
         a.rope = k_new != nullptr ? 1 : 0;
-        if (a.rope && workspace_fits(st, 0)) {  // (without one the launch computes cos and sin itself)
+        if (a.rope && workspace_present(st)) {  // (without one the launch computes cos and sin itself)
             uint32_t* counters = nullptr;
             void* general = nullptr;
             const int32_t status = workspace_counters(st, 0, 0, &general, &counters);

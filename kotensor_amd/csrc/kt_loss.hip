@@ -221,7 +221,9 @@ extern "C" int32_t kt_fused_cross_entropy(const float* hidden, int32_t rows, con
     // the stream's kept area; an allocation of this call where there is none (67 MB allocated
     // and freed on every call cost 50 to 250 us)
     void* scratch = nullptr;
-    if ((status = loss_area(st, bytes, &scratch))) return status;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    KT_HIP(hipStreamIsCapturing(st, &capture));
+    if (capture == hipStreamCaptureStatusNone && (status = call_area(CALL_LOSS, st, bytes, LOSS_LIMIT, &scratch))) return status;
     const bool allocated = scratch == nullptr;
     if (allocated) KT_HIP(hipMallocAsync(&scratch, bytes, st));
     float* logits = static_cast<float*>(scratch);
@@ -273,7 +275,7 @@ extern "C" int32_t kt_fused_cross_entropy(const float* hidden, int32_t rows, con
     }();
     hipError_t freed = hipSuccess;
     if (allocated) freed = hipFreeAsync(scratch, st);
-    else loss_area_done(st);
+    else call_area_done(CALL_LOSS, st);
     if (status) return status;
     if (freed != hipSuccess) return hip_fail(freed, "hipFreeAsync");
     return KT_OK;

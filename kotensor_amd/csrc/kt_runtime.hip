@@ -36,13 +36,13 @@ struct Block {
     size_t bytes = 0;       // whole allocation
     size_t zbytes = 0;      // the zeroed accumulator region after the counters
     bool captured = false;  // handed to a kernel recorded into a graph
-    bool busy = false;      // a loss area handed to a call that is still enqueuing
+    bool busy = false;      // a call area whose call is still enqueuing
     int32_t fault = -1;     // the stream's slot of the fault words, once a kernel took it
 };
 std::mutex g_ws_mutex;
 std::map<std::pair<int, hipStream_t>, Block> g_ws;
-// The fused loss's areas, beside the workspaces its products use (loss_area).
-std::map<std::pair<int, hipStream_t>, Block> g_loss;
+// The areas one enqueuing call holds at a time, per kind (call_area).
+std::map<std::pair<int, hipStream_t>, Block> g_areas[CALL_AREAS];
 // Blocks replaced or orphaned while a recorded graph may still address them. A graph
 // keeps the addresses it was recorded with, and graphs can outlive their stream, so
 // these stay allocated until the process ends (each is smaller than its successor, so
@@ -138,49 +138,58 @@ int32_t workspace(hipStream_t stream, size_t bytes, void** out) {
     return KT_OK;
 }
 
-bool workspace_fits(hipStream_t stream, size_t bytes) {
-    if (t_fixed) return bytes <= t_fixed->bytes - COUNTER_BYTES - t_fixed->zero_bytes;
+bool workspace_present(hipStream_t stream) {
+    if (t_fixed) return true;
     int device = 0;
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (hipGetDevice(&device) != hipSuccess || hipStreamIsCapturing(stream, &capture) != hipSuccess) return false;
     if (capture == hipStreamCaptureStatusNone) return true;
     std::lock_guard<std::mutex> lock(g_ws_mutex);
     const auto it = g_ws.find(std::make_pair(device, stream));
-    return it != g_ws.end() && it->second.ptr && COUNTER_BYTES + it->second.zbytes + bytes <= it->second.bytes;
+    return it != g_ws.end() && it->second.ptr;
 }
 
-int32_t loss_area(hipStream_t stream, size_t bytes, void** out) {
+int32_t call_area(CallArea kind, hipStream_t stream, size_t bytes, size_t limit, void** out) {
     *out = nullptr;
-    if (bytes > LOSS_AREA_BYTES) return KT_OK;
+    if (bytes > limit) return KT_OK;
+    if (t_fixed) {  // the fixed workspace's general area, where it is large enough
+        const size_t head = COUNTER_BYTES + t_fixed->zero_bytes;
+        if (bytes <= t_fixed->bytes - head) *out = t_fixed->ptr + head;
+        return KT_OK;
+    }
     int device = 0;
     KT_HIP(hipGetDevice(&device));
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     KT_HIP(hipStreamIsCapturing(stream, &capture));
-    if (capture != hipStreamCaptureStatusNone) return KT_OK;
+    const bool capturing = capture != hipStreamCaptureStatusNone;
     std::lock_guard<std::mutex> lock(g_ws_mutex);
-    Block& b = g_loss[std::make_pair(device, stream)];
+    if (capturing && g_areas[kind].find(std::make_pair(device, stream)) == g_areas[kind].end()) return KT_OK;
+    Block& b = g_areas[kind][std::make_pair(device, stream)];
     if (b.busy) return KT_OK;  // another thread is enqueuing with it
     if (b.bytes < bytes) {
+        if (capturing) return KT_OK;
         if (b.ptr) {
             KT_HIP(hipStreamSynchronize(stream));
-            KT_HIP(hipFree(b.ptr));
+            if (b.captured) g_retired.push_back(b.ptr);  // a graph may still address it
+            else KT_HIP(hipFree(b.ptr));
             b = Block{};
         }
-        const size_t want = bytes + bytes / 4 < LOSS_AREA_BYTES ? bytes + bytes / 4 : LOSS_AREA_BYTES;
+        const size_t want = bytes + bytes / 4 < limit ? bytes + bytes / 4 : limit;
         KT_HIP(hipMalloc(&b.ptr, want));
         b.bytes = want;
     }
+    if (capturing) b.captured = true;
     b.busy = true;
     *out = b.ptr;
     return KT_OK;
 }
 
-void loss_area_done(hipStream_t stream) {
+void call_area_done(CallArea kind, hipStream_t stream) {
     int device = 0;
-    if (hipGetDevice(&device) != hipSuccess) return;
+    if (t_fixed || hipGetDevice(&device) != hipSuccess) return;
     std::lock_guard<std::mutex> lock(g_ws_mutex);
-    const auto it = g_loss.find(std::make_pair(device, stream));
-    if (it != g_loss.end()) it->second.busy = false;
+    const auto it = g_areas[kind].find(std::make_pair(device, stream));
+    if (it != g_areas[kind].end()) it->second.busy = false;
 }
 
 int32_t workspace_counters(hipStream_t stream, size_t bytes, size_t count, void** general, uint32_t** counters) {
@@ -507,10 +516,12 @@ int32_t kt_stream_destroy(void* stream) {
             else if (it->second.ptr) KT_HIP(hipFree(it->second.ptr));
             g_ws.erase(it);
         }
-        const auto loss = g_loss.find(std::make_pair(device, s));
-        if (loss != g_loss.end()) {
-            if (loss->second.ptr) KT_HIP(hipFree(loss->second.ptr));
-            g_loss.erase(loss);
+        for (auto& areas : g_areas) {
+            const auto area = areas.find(std::make_pair(device, s));
+            if (area == areas.end()) continue;
+            if (area->second.ptr && area->second.captured) g_retired.push_back(area->second.ptr);
+            else if (area->second.ptr) KT_HIP(hipFree(area->second.ptr));
+            areas.erase(area);
         }
     }
     KT_HIP(hipStreamDestroy(s));

@@ -680,14 +680,22 @@ int32_t launch_slices_reduce(const float* part, int32_t splits, int32_t m, int32
     return KT_OK;
 }
 
-// Slices of `steps` for a grid of `tiles` workgroups: two workgroups per CU, as many slices
-// as the workspace holds (none of it: one slice). slice: bytes of a slice's sums.
-int32_t choose_slices(hipStream_t st, int64_t tiles, int32_t steps, size_t slice, int32_t* per_slice) {
-    int64_t splits = (2 * cu_count() + tiles - 1) / tiles;
-    splits = std::min<int64_t>(std::min<int64_t>(splits, MAX_SPLITS), steps);
-    if (splits > 1 && !workspace_fits(st, splits * slice)) splits = 1;
-    *per_slice = ceil_div(steps, static_cast<int32_t>(splits));
-    return ceil_div(steps, *per_slice);
+// Slices of `steps` for a grid of `tiles` workgroups: two workgroups per CU, and the area for
+// their sums (slice: bytes of one); one slice, which needs none, where there is no area.
+int32_t choose_slices(hipStream_t st, int64_t tiles, int32_t steps, size_t slice, int32_t* splits, int32_t* per_slice,
+                      void** area) {
+    int64_t want = (2 * cu_count() + tiles - 1) / tiles;
+    want = std::min<int64_t>(std::min<int64_t>(want, MAX_SPLITS), steps);
+    *per_slice = ceil_div(steps, static_cast<int32_t>(want));
+    *splits = ceil_div(steps, *per_slice);
+    *area = nullptr;
+    if (*splits == 1) return KT_OK;
+    const int32_t status = call_area(CALL_SLICES, st, *splits * slice, SLICES_LIMIT, area);
+    if (!*area) {
+        *splits = 1;
+        *per_slice = steps;
+    }
+    return status;
 }
 
 template <int BITS, bool ZP, int WM>
@@ -734,20 +742,16 @@ int32_t launch_transposed_split(const float* dy, int32_t m, const WeightView& w,
     const int64_t tiles = static_cast<int64_t>(p.tiles_m) * ceil_div(w.K, 128 * (4 / wm));
     p.steps = ceil_div(w.bpr, w.bits == 4 ? 32 : 64);
     const size_t slice = static_cast<size_t>(m) * w.K * sizeof(float);
-    p.splits = choose_slices(st, tiles, p.steps, slice, &p.steps_per_split);
+    const int64_t max_blocks = tiles * MAX_SPLITS;
+    if (max_blocks > INT32_MAX) return fail(KT_ERR_SHAPE, "grid of %lld blocks is out of range", static_cast<long long>(max_blocks));
+    void* area = nullptr;
+    if (const int32_t status = choose_slices(st, tiles, p.steps, slice, &p.splits, &p.steps_per_split, &area)) return status;
+    if (area) p.out = static_cast<float*>(area);
     // Runs: no longer a sequence of sums than the row-by-row kernel's N / 256, or 16 steps
     // (28 steps in one run at N = 3584 had 1.19e-7 of the 2-norm against its 1.04e-7, two
     // runs of 14 have 1.01e-7; each run after a slice's first takes about 7 us).
     p.run = ceil_div(p.steps_per_split, ceil_div(p.steps_per_split, std::max(16, p.steps / 4)));
-    if (p.splits > 1) {
-        void* ws = nullptr;
-        const int32_t status = workspace(st, p.splits * slice, &ws);
-        if (status) return status;
-        p.out = static_cast<float*>(ws);
-    }
-    const int64_t blocks64 = tiles * p.splits;
-    if (blocks64 > INT32_MAX) return fail(KT_ERR_SHAPE, "grid of %lld blocks is out of range", static_cast<long long>(blocks64));
-    const uint32_t blocks = static_cast<uint32_t>(blocks64);
+    const uint32_t blocks = static_cast<uint32_t>(tiles * p.splits);
     if (w.bits == 4)
         wm == 4   ? launch_transposed_tiles<4, 4>(p, blocks, st)
         : wm == 2 ? launch_transposed_tiles<4, 2>(p, blocks, st)
@@ -756,8 +760,13 @@ int32_t launch_transposed_split(const float* dy, int32_t m, const WeightView& w,
         wm == 4   ? launch_transposed_tiles<8, 4>(p, blocks, st)
         : wm == 2 ? launch_transposed_tiles<8, 2>(p, blocks, st)
                   : launch_transposed_tiles<8, 1>(p, blocks, st);
-    KT_LAUNCHED("qmatmul_transposed: split kernel");
-    return p.splits > 1 ? launch_slices_reduce(p.out, p.splits, m, w.K, dx, accumulate, 1.0f, nullptr, st) : KT_OK;
+    const hipError_t err = hipGetLastError();
+    int32_t status = err == hipSuccess ? KT_OK : hip_fail(err, "qmatmul_transposed: split kernel");
+    if (area) {
+        if (status == KT_OK) status = launch_slices_reduce(p.out, p.splits, m, w.K, dx, accumulate, 1.0f, nullptr, st);
+        call_area_done(CALL_SLICES, st);
+    }
+    return status;
 }
 
 // generic_matmul (kt_misc.hip: one thread per output, k in sequence) stays where the product
@@ -777,21 +786,22 @@ int32_t launch_forward_split(const float* a, int32_t m, const WeightView& w, flo
     const int64_t tiles = static_cast<int64_t>(p.tiles_m) * ceil_div(w.bpr, (w.bits == 4 ? 64 : 128) * (4 / wm));
     p.steps = ceil_div(w.K, STEP);
     const size_t slice = static_cast<size_t>(m) * w.N * sizeof(float);
-    p.splits = choose_slices(st, tiles, p.steps, slice, &p.steps_per_split);
-    if (p.splits > 1) {
-        void* ws = nullptr;
-        const int32_t status = workspace(st, p.splits * slice, &ws);
-        if (status) return status;
-        p.c = static_cast<float*>(ws);
-    }
-    const int64_t blocks64 = tiles * p.splits;
-    if (blocks64 > INT32_MAX) return fail(KT_ERR_SHAPE, "grid of %lld blocks is out of range", static_cast<long long>(blocks64));
-    const uint32_t blocks = static_cast<uint32_t>(blocks64);
+    const int64_t max_blocks = tiles * MAX_SPLITS;
+    if (max_blocks > INT32_MAX) return fail(KT_ERR_SHAPE, "grid of %lld blocks is out of range", static_cast<long long>(max_blocks));
+    void* area = nullptr;
+    if (const int32_t status = choose_slices(st, tiles, p.steps, slice, &p.splits, &p.steps_per_split, &area)) return status;
+    if (area) p.c = static_cast<float*>(area);
+    const uint32_t blocks = static_cast<uint32_t>(tiles * p.splits);
     if (w.bits == 4) launch_forward_rows<4, true>(wm, p, blocks, st);
     else if (w.z) launch_forward_rows<8, true>(wm, p, blocks, st);
     else launch_forward_rows<8, false>(wm, p, blocks, st);
-    KT_LAUNCHED("qmatmul: split kernel");
-    return p.splits > 1 ? launch_slices_reduce(p.c, p.splits, m, w.N, c, accumulate, alpha, bias, st) : KT_OK;
+    const hipError_t err = hipGetLastError();
+    int32_t status = err == hipSuccess ? KT_OK : hip_fail(err, "qmatmul: split kernel");
+    if (area) {
+        if (status == KT_OK) status = launch_slices_reduce(p.c, p.splits, m, w.N, c, accumulate, alpha, bias, st);
+        call_area_done(CALL_SLICES, st);
+    }
+    return status;
 }
 
 }  // namespace kt

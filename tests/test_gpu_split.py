@@ -177,3 +177,38 @@ def test_transposed_recorded_without_workspace(kt, oracle_lib):
         stream.synchronize()
         _lib.call("kt_graph_destroy", graph)
         stream.destroy()
+
+
+def test_two_threads_on_one_stream(kt, oracle_lib):
+    """Two threads call the sliced products on the null stream at once: the slices' area
+    belongs to one enqueuing call at a time (the other runs one slice)."""
+    import threading
+
+    operands = []
+    for i, (m, k, n) in enumerate([(5, 4096, 1023), (40, 3000, 515)]):
+        q = _weights(oracle_lib, k, n, 4, 64, 40 + i)
+        rng = np.random.default_rng(50 + i)
+        x, dy = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((m, n)).astype(np.float32)
+        w = q.dequantize().astype(np.float64)
+        operands.append((x, dy, upload_quantized(kt, q), x @ w, dy @ w.T))
+    errors = [[], []]
+
+    def work(i):
+        x, dy, qt, y, dx = operands[i]
+        m, (k, n) = x.shape[0], qt.shape
+        a, b = kt.DeviceBuffer.from_numpy(x), kt.DeviceBuffer.from_numpy(dy)
+        outs = [(kt.DeviceBuffer(m * n * 4), kt.DeviceBuffer(m * k * 4)) for _ in range(40)]
+        for c, d in outs:
+            kt.MatMul.multiply_quantized(a, qt, c, m, accumulate=False)
+            kt.MatMul.multiply_by_quantized_transposed(b, qt, d, m, accumulate=False)
+        kt.synchronize()
+        for c, d in outs:
+            errors[i] += [normwise_rel(c.download(np.float32).reshape(m, n), y), normwise_rel(d.download(np.float32).reshape(m, k), dx)]
+
+    banner("split-two-threads")
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert all(len(e) == 80 and max(e) <= TOL for e in errors)
