@@ -67,8 +67,8 @@ bool workspace_present(hipStream_t stream);
 
 // An area of the stream that one call holds while it enqueues its launches (two threads on
 // one stream then never interleave launches on it), kept for the next call and freed with the
-// stream; nullptr where the call does without: more than `limit` bytes, another thread's call
-// in progress, a captured stream whose area is too small. (Calls on a caller's fixed
+// stream; nullptr where the call does without: more than `limit` bytes, no memory left, another
+// thread's call in progress, a captured stream whose area is too small. (Calls on a caller's fixed
 // workspace get its general area.) The
 // split products' slices and the prefill attention's parts are CALL_SLICES; the fused loss's
 // scratch is CALL_LOSS, since its products want the other. A call that got one returns it
