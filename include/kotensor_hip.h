@@ -140,7 +140,13 @@ int32_t kt_debug_wait_limits(uint32_t spin_limit, int32_t withhold);
  * or recorded for it. A workspace that a graph addresses is never freed before the
  * process ends, even when a later call grows it or the stream is destroyed. Replays
  * and eager calls that share a workspace must not run concurrently: replay a graph on
- * the stream it was recorded on, or keep that stream idle during the replay. */
+ * the stream it was recorded on, or keep that stream idle during the replay.
+ * The calls that need no such workspace (kt_qmatmul_transposed, products of odd widths,
+ * kt_attention of 16 and more tokens) may hold scratch of their own: recorded, it belongs
+ * to the graph and kt_graph_destroy frees it, so their replays on any stream are
+ * independent of eager calls and of other graphs (as for any graph, two replays of one
+ * graph write the same outputs and are the caller's to order). A capture begun by other
+ * means records them without scratch. */
 int32_t kt_graph_begin(void* stream);
 int32_t kt_graph_end(void* stream, void** graph);
 int32_t kt_graph_launch(void* graph, void* stream);

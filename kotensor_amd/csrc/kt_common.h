@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <memory>
+
 #include "../../include/kotensor_hip.h"
 
 namespace kt {
@@ -65,17 +67,34 @@ WaitLimits wait_limits();
 // not), for calls that have a way to do without its counter region.
 bool workspace_present(hipStream_t stream);
 
-// An area of the stream that one call holds while it enqueues its launches (two threads on
-// one stream then never interleave launches on it), kept for the next call and freed with the
-// stream; nullptr where the call does without: more than `limit` bytes, no memory left, another
-// thread's call in progress, a captured stream whose area is too small. (Calls on a caller's fixed
-// workspace get its general area.) The
+// Scratch that one call holds while it enqueues its launches (two threads on one stream then
+// never interleave launches on it). An eager call takes the area of its stream, which stays for
+// the next call and is freed with the stream; a call recorded between kt_graph_begin and
+// kt_graph_end takes one that belongs to the graph (calls recorded on one stream share it, in
+// stream order) and is freed with it, so that replays on any stream and eager calls never meet
+// in it. ptr stays null where the call does without: more than `limit` bytes, no memory left,
+// another thread's call in progress, a capture begun by other means, whose graph's end the
+// library does not see. (Calls on a caller's fixed workspace get its general area.) The
 // split products' slices and the prefill attention's parts are CALL_SLICES; the fused loss's
-// scratch is CALL_LOSS, since its products want the other. A call that got one returns it
-// with call_area_done once its last launch is enqueued.
+// scratch is CALL_LOSS, since its products want the other.
 enum CallArea { CALL_SLICES, CALL_LOSS, CALL_AREAS };
-int32_t call_area(CallArea kind, hipStream_t stream, size_t bytes, size_t limit, void** out);
-void call_area_done(CallArea kind, hipStream_t stream);
+struct Area {
+    void* ptr = nullptr;
+    size_t bytes = 0;
+    bool busy = false;  // its call is still enqueuing
+};
+class CallScratch {
+  public:
+    CallScratch() = default;
+    CallScratch(const CallScratch&) = delete;
+    CallScratch& operator=(const CallScratch&) = delete;
+    ~CallScratch();  // after the call's last launch is enqueued
+    int32_t take(CallArea kind, hipStream_t stream, size_t bytes, size_t limit);
+    void* ptr = nullptr;
+
+  private:
+    std::shared_ptr<Area> held_;
+};
 constexpr size_t SLICES_LIMIT = size_t(64) << 20;
 constexpr size_t LOSS_LIMIT = size_t(192) << 20;
 

@@ -1570,14 +1570,11 @@ static int32_t attention_launch(const float* q, int32_t tokens, const int32_t* p
         const size_t parts_bytes = static_cast<size_t>(num_kv_heads) * 2 * ceil_div(key_bound, PKT) *
                                    (head_dim == 64 ? parts_block_bytes(64) : parts_block_bytes(128));
         if (key_bound >= PARTS_MIN_KEYS && G <= SPLIT_ROWS) {
-            void* parts = nullptr;
-            if (const int32_t status = call_area(CALL_SLICES, st, parts_bytes, SLICES_LIMIT, &parts)) return status;
-            if (parts) {
-                const int32_t status = head_dim == 64 ? launch_prefill_parts<64>(a, tokens, key_bound, static_cast<uint8_t*>(parts), st)
-                                                      : launch_prefill_parts<128>(a, tokens, key_bound, static_cast<uint8_t*>(parts), st);
-                call_area_done(CALL_SLICES, st);
-                return status;
-            }
+            CallScratch parts;
+            if (const int32_t status = parts.take(CALL_SLICES, st, parts_bytes, SLICES_LIMIT)) return status;
+            if (parts.ptr)
+                return head_dim == 64 ? launch_prefill_parts<64>(a, tokens, key_bound, static_cast<uint8_t*>(parts.ptr), st)
+                                      : launch_prefill_parts<128>(a, tokens, key_bound, static_cast<uint8_t*>(parts.ptr), st);
         }
         const int32_t qb_tokens = PQ_ROWS / G;
         const int32_t nqb = ceil_div(tokens, qb_tokens);

@@ -220,12 +220,12 @@ extern "C" int32_t kt_fused_cross_entropy(const float* hidden, int32_t rows, con
     const size_t bytes = logit_bytes + 2 * row_bytes + static_cast<size_t>(active) * (sizeof(float) + 2 * sizeof(int32_t));
     // the stream's kept area; an allocation of this call where there is none (67 MB allocated
     // and freed on every call cost 50 to 250 us)
-    void* scratch = nullptr;
+    CallScratch kept;
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     KT_HIP(hipStreamIsCapturing(st, &capture));
-    if (capture == hipStreamCaptureStatusNone && (status = call_area(CALL_LOSS, st, bytes, LOSS_LIMIT, &scratch))) return status;
-    const bool allocated = scratch == nullptr;
-    if (allocated) KT_HIP(hipMallocAsync(&scratch, bytes, st));
+    if (capture == hipStreamCaptureStatusNone && (status = kept.take(CALL_LOSS, st, bytes, LOSS_LIMIT))) return status;
+    void* scratch = kept.ptr;
+    if (!kept.ptr) KT_HIP(hipMallocAsync(&scratch, bytes, st));
     float* logits = static_cast<float*>(scratch);
     float* inputs = reinterpret_cast<float*>(static_cast<char*>(scratch) + logit_bytes);
     float* pass_grad = reinterpret_cast<float*>(static_cast<char*>(scratch) + logit_bytes + row_bytes);
@@ -274,8 +274,7 @@ extern "C" int32_t kt_fused_cross_entropy(const float* hidden, int32_t rows, con
         return KT_OK;
     }();
     hipError_t freed = hipSuccess;
-    if (allocated) freed = hipFreeAsync(scratch, st);
-    else call_area_done(CALL_LOSS, st);
+    if (!kept.ptr) freed = hipFreeAsync(scratch, st);
     if (status) return status;
     if (freed != hipSuccess) return hip_fail(freed, "hipFreeAsync");
     return KT_OK;

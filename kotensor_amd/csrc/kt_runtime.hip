@@ -36,13 +36,21 @@ struct Block {
     size_t bytes = 0;       // whole allocation
     size_t zbytes = 0;      // the zeroed accumulator region after the counters
     bool captured = false;  // handed to a kernel recorded into a graph
-    bool busy = false;      // a call area whose call is still enqueuing
     int32_t fault = -1;     // the stream's slot of the fault words, once a kernel took it
 };
 std::mutex g_ws_mutex;
 std::map<std::pair<int, hipStream_t>, Block> g_ws;
-// The areas one enqueuing call holds at a time, per kind (call_area).
-std::map<std::pair<int, hipStream_t>, Block> g_areas[CALL_AREAS];
+// The areas of the streams' eager calls, per kind (CallScratch).
+std::map<std::pair<int, hipStream_t>, std::shared_ptr<Area>> g_areas[CALL_AREAS];
+// The areas of recorded calls, while their capture runs (by its id) and once it is a graph:
+// the graph's end frees them.
+struct Capture {
+    hipStream_t origin = nullptr;                          // the stream of kt_graph_begin
+    std::map<std::pair<int, hipStream_t>, std::shared_ptr<Area>> areas;  // by kind and stream
+    std::vector<void*> blocks;                             // all that the recorded calls may address
+};
+std::map<unsigned long long, Capture> g_captures;
+std::map<hipGraphExec_t, std::vector<void*>> g_graph_blocks;
 // Blocks replaced or orphaned while a recorded graph may still address them. A graph
 // keeps the addresses it was recorded with, and graphs can outlive their stream, so
 // these stay allocated until the process ends (each is smaller than its successor, so
@@ -149,51 +157,74 @@ bool workspace_present(hipStream_t stream) {
     return it != g_ws.end() && it->second.ptr;
 }
 
-int32_t call_area(CallArea kind, hipStream_t stream, size_t bytes, size_t limit, void** out) {
-    *out = nullptr;
+namespace {
+// hipMalloc and hipFree while this thread may be capturing: they touch no captured stream.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const hipError_t err = hipThreadExchangeStreamCaptureMode(&mode);
+    ~RelaxedCapture() {
+        if (err == hipSuccess) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+};
+
+// Frees a graph's blocks (hipFree waits for the device, so for replays in flight).
+void free_blocks(const std::vector<void*>& blocks) {
+    if (blocks.empty()) return;
+    RelaxedCapture relaxed;
+    for (void* b : blocks)
+        if (hipFree(b) != hipSuccess) (void)hipGetLastError();
+}
+}  // namespace
+
+int32_t CallScratch::take(CallArea kind, hipStream_t stream, size_t bytes, size_t limit) {
     if (bytes > limit) return KT_OK;
     if (t_fixed) {  // the fixed workspace's general area, where it is large enough
         const size_t head = COUNTER_BYTES + t_fixed->zero_bytes;
-        if (bytes <= t_fixed->bytes - head) *out = t_fixed->ptr + head;
+        if (bytes <= t_fixed->bytes - head) ptr = t_fixed->ptr + head;
         return KT_OK;
     }
     int device = 0;
     KT_HIP(hipGetDevice(&device));
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    KT_HIP(hipStreamIsCapturing(stream, &capture));
-    const bool capturing = capture != hipStreamCaptureStatusNone;
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    KT_HIP(hipStreamGetCaptureInfo(stream, &status, &id));
     std::lock_guard<std::mutex> lock(g_ws_mutex);
-    if (capturing && g_areas[kind].find(std::make_pair(device, stream)) == g_areas[kind].end()) return KT_OK;
-    Block& b = g_areas[kind][std::make_pair(device, stream)];
-    if (b.busy) return KT_OK;  // another thread is enqueuing with it
-    if (b.bytes < bytes) {
-        if (capturing) return KT_OK;
-        if (b.ptr) {
+    Capture* capture = nullptr;
+    if (status != hipStreamCaptureStatusNone) {
+        const auto it = g_captures.find(id);
+        if (it == g_captures.end()) return KT_OK;
+        capture = &it->second;
+    }
+    std::shared_ptr<Area>& area = capture ? capture->areas[std::make_pair(static_cast<int>(kind), stream)]
+                                          : g_areas[kind][std::make_pair(device, stream)];
+    if (!area) area = std::make_shared<Area>();
+    if (area->busy) return KT_OK;  // another thread is enqueuing with it
+    if (area->bytes < bytes) {
+        if (area->ptr && !capture) {
             KT_HIP(hipStreamSynchronize(stream));
-            if (b.captured) g_retired.push_back(b.ptr);  // a graph may still address it
-            else KT_HIP(hipFree(b.ptr));
-            b = Block{};
+            KT_HIP(hipFree(area->ptr));
         }
+        *area = Area{};
         const size_t want = bytes + bytes / 4 < limit ? bytes + bytes / 4 : limit;
-        if (hipMalloc(&b.ptr, want) != hipSuccess) {  // no memory left: the call does without
+        RelaxedCapture relaxed;
+        if (hipMalloc(&area->ptr, want) != hipSuccess) {  // no memory left: the call does without
             (void)hipGetLastError();
-            b = Block{};
+            area->ptr = nullptr;
             return KT_OK;
         }
-        b.bytes = want;
+        if (capture) capture->blocks.push_back(area->ptr);
+        area->bytes = want;
     }
-    if (capturing) b.captured = true;
-    b.busy = true;
-    *out = b.ptr;
+    area->busy = true;
+    held_ = area;
+    ptr = area->ptr;
     return KT_OK;
 }
 
-void call_area_done(CallArea kind, hipStream_t stream) {
-    int device = 0;
-    if (t_fixed || hipGetDevice(&device) != hipSuccess) return;
+CallScratch::~CallScratch() {
+    if (!held_) return;
     std::lock_guard<std::mutex> lock(g_ws_mutex);
-    const auto it = g_areas[kind].find(std::make_pair(device, stream));
-    if (it != g_areas[kind].end()) it->second.busy = false;
+    held_->busy = false;
 }
 
 int32_t workspace_counters(hipStream_t stream, size_t bytes, size_t count, void** general, uint32_t** counters) {
@@ -523,8 +554,7 @@ int32_t kt_stream_destroy(void* stream) {
         for (auto& areas : g_areas) {
             const auto area = areas.find(std::make_pair(device, s));
             if (area == areas.end()) continue;
-            if (area->second.ptr && area->second.captured) g_retired.push_back(area->second.ptr);
-            else if (area->second.ptr) KT_HIP(hipFree(area->second.ptr));
+            if (area->second->ptr) KT_HIP(hipFree(area->second->ptr));
             areas.erase(area);
         }
     }
@@ -545,19 +575,50 @@ int32_t kt_debug_wait_limits(uint32_t spin_limit, int32_t withhold) {
 
 int32_t kt_graph_begin(void* stream) {
     if (!stream) return fail(KT_ERR_ARGUMENT, "the null stream cannot be captured; create a stream");
-    KT_HIP(hipStreamBeginCapture(static_cast<hipStream_t>(stream), hipStreamCaptureModeThreadLocal));
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    KT_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (hipStreamGetCaptureInfo(st, &status, &id) == hipSuccess && status == hipStreamCaptureStatusActive) {
+        std::lock_guard<std::mutex> lock(g_ws_mutex);
+        g_captures[id].origin = st;
+    }
     return KT_OK;
 }
 
 int32_t kt_graph_end(void* stream, void** graph) {
     if (!stream || !graph) return fail(KT_ERR_ARGUMENT, "stream or graph is NULL");
     *graph = nullptr;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    std::vector<void*> blocks;  // of the calls recorded since kt_graph_begin
+    {
+        std::lock_guard<std::mutex> lock(g_ws_mutex);
+        for (auto it = g_captures.begin(); it != g_captures.end();) {
+            if (it->second.origin != st) {
+                ++it;
+                continue;
+            }
+            blocks.insert(blocks.end(), it->second.blocks.begin(), it->second.blocks.end());
+            it = g_captures.erase(it);
+        }
+    }
     hipGraph_t g = nullptr;
-    KT_HIP(hipStreamEndCapture(static_cast<hipStream_t>(stream), &g));
+    hipError_t err = hipStreamEndCapture(st, &g);
+    if (err != hipSuccess) {
+        free_blocks(blocks);
+        return hip_fail(err, "hipStreamEndCapture");
+    }
     hipGraphExec_t exec = nullptr;
-    const hipError_t err = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
+    err = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
     (void)hipGraphDestroy(g);
-    if (err != hipSuccess) return hip_fail(err, "hipGraphInstantiate");
+    if (err != hipSuccess) {
+        free_blocks(blocks);
+        return hip_fail(err, "hipGraphInstantiate");
+    }
+    if (!blocks.empty()) {
+        std::lock_guard<std::mutex> lock(g_ws_mutex);
+        g_graph_blocks[exec] = std::move(blocks);
+    }
     *graph = exec;
     return KT_OK;
 }
@@ -569,7 +630,20 @@ int32_t kt_graph_launch(void* graph, void* stream) {
 }
 
 int32_t kt_graph_destroy(void* graph) {
-    if (graph) KT_HIP(hipGraphExecDestroy(static_cast<hipGraphExec_t>(graph)));
+    if (!graph) return KT_OK;
+    const hipGraphExec_t exec = static_cast<hipGraphExec_t>(graph);
+    std::vector<void*> blocks;
+    {
+        std::lock_guard<std::mutex> lock(g_ws_mutex);
+        const auto it = g_graph_blocks.find(exec);
+        if (it != g_graph_blocks.end()) {
+            blocks = std::move(it->second);
+            g_graph_blocks.erase(it);
+        }
+    }
+    const hipError_t err = hipGraphExecDestroy(exec);
+    free_blocks(blocks);
+    if (err != hipSuccess) return hip_fail(err, "hipGraphExecDestroy");
     return KT_OK;
 }
 

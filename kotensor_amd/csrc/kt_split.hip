@@ -683,15 +683,14 @@ int32_t launch_slices_reduce(const float* part, int32_t splits, int32_t m, int32
 // Slices of `steps` for a grid of `tiles` workgroups: two workgroups per CU, and the area for
 // their sums (slice: bytes of one); one slice, which needs none, where there is no area.
 int32_t choose_slices(hipStream_t st, int64_t tiles, int32_t steps, size_t slice, int32_t* splits, int32_t* per_slice,
-                      void** area) {
+                      CallScratch* area) {
     int64_t want = (2 * cu_count() + tiles - 1) / tiles;
     want = std::min<int64_t>(std::min<int64_t>(want, MAX_SPLITS), steps);
     *per_slice = ceil_div(steps, static_cast<int32_t>(want));
     *splits = ceil_div(steps, *per_slice);
-    *area = nullptr;
     if (*splits == 1) return KT_OK;
-    const int32_t status = call_area(CALL_SLICES, st, *splits * slice, SLICES_LIMIT, area);
-    if (!*area) {
+    const int32_t status = area->take(CALL_SLICES, st, *splits * slice, SLICES_LIMIT);
+    if (!area->ptr) {
         *splits = 1;
         *per_slice = steps;
     }
@@ -744,9 +743,9 @@ int32_t launch_transposed_split(const float* dy, int32_t m, const WeightView& w,
     const size_t slice = static_cast<size_t>(m) * w.K * sizeof(float);
     const int64_t max_blocks = tiles * MAX_SPLITS;
     if (max_blocks > INT32_MAX) return fail(KT_ERR_SHAPE, "grid of %lld blocks is out of range", static_cast<long long>(max_blocks));
-    void* area = nullptr;
+    CallScratch area;
     if (const int32_t status = choose_slices(st, tiles, p.steps, slice, &p.splits, &p.steps_per_split, &area)) return status;
-    if (area) p.out = static_cast<float*>(area);
+    if (area.ptr) p.out = static_cast<float*>(area.ptr);
     // Runs: no longer a sequence of sums than the row-by-row kernel's N / 256, or 16 steps
     // (28 steps in one run at N = 3584 had 1.19e-7 of the 2-norm against its 1.04e-7, two
     // runs of 14 have 1.01e-7; each run after a slice's first takes about 7 us).
@@ -762,10 +761,7 @@ int32_t launch_transposed_split(const float* dy, int32_t m, const WeightView& w,
                   : launch_transposed_tiles<8, 1>(p, blocks, st);
     const hipError_t err = hipGetLastError();
     int32_t status = err == hipSuccess ? KT_OK : hip_fail(err, "qmatmul_transposed: split kernel");
-    if (area) {
-        if (status == KT_OK) status = launch_slices_reduce(p.out, p.splits, m, w.K, dx, accumulate, 1.0f, nullptr, st);
-        call_area_done(CALL_SLICES, st);
-    }
+    if (area.ptr && status == KT_OK) status = launch_slices_reduce(p.out, p.splits, m, w.K, dx, accumulate, 1.0f, nullptr, st);
     return status;
 }
 
@@ -788,19 +784,16 @@ int32_t launch_forward_split(const float* a, int32_t m, const WeightView& w, flo
     const size_t slice = static_cast<size_t>(m) * w.N * sizeof(float);
     const int64_t max_blocks = tiles * MAX_SPLITS;
     if (max_blocks > INT32_MAX) return fail(KT_ERR_SHAPE, "grid of %lld blocks is out of range", static_cast<long long>(max_blocks));
-    void* area = nullptr;
+    CallScratch area;
     if (const int32_t status = choose_slices(st, tiles, p.steps, slice, &p.splits, &p.steps_per_split, &area)) return status;
-    if (area) p.c = static_cast<float*>(area);
+    if (area.ptr) p.c = static_cast<float*>(area.ptr);
     const uint32_t blocks = static_cast<uint32_t>(tiles * p.splits);
     if (w.bits == 4) launch_forward_rows<4, true>(wm, p, blocks, st);
     else if (w.z) launch_forward_rows<8, true>(wm, p, blocks, st);
     else launch_forward_rows<8, false>(wm, p, blocks, st);
     const hipError_t err = hipGetLastError();
     int32_t status = err == hipSuccess ? KT_OK : hip_fail(err, "qmatmul: split kernel");
-    if (area) {
-        if (status == KT_OK) status = launch_slices_reduce(p.c, p.splits, m, w.N, c, accumulate, alpha, bias, st);
-        call_area_done(CALL_SLICES, st);
-    }
+    if (area.ptr && status == KT_OK) status = launch_slices_reduce(p.c, p.splits, m, w.N, c, accumulate, alpha, bias, st);
     return status;
 }
 

@@ -1,0 +1,151 @@
+"""Calls with scratch of their own (split products, prompt attention on parts) recorded into
+graphs: the graph has its own scratch, so replays on any stream, next to eager calls or to
+other graphs' replays, give the eager call's bits."""
+import contextlib
+import ctypes
+
+import numpy as np
+import pytest
+
+from gpu_helpers import banner, same_bits, upload_quantized
+
+pytestmark = pytest.mark.gpu
+
+
+class _Call:
+    """One call on operands of its own: run() enqueues it, result() downloads its output."""
+
+    def __init__(self, kt, shape):
+        self.kt, self.out = kt, kt.DeviceBuffer(int(np.prod(shape)) * 4)
+
+    def result(self):
+        return self.out.download(np.float32)
+
+    def eager(self):
+        self.out.fill_zero()
+        self.run(None)
+        self.kt.synchronize()
+        return self.result()
+
+
+class _Transposed(_Call):
+    def __init__(self, kt, oracle_lib, m, k, n, seed):
+        super().__init__(kt, (m, k))
+        rng = np.random.default_rng(seed)
+        st, q = oracle_lib.quantize((rng.standard_normal((k, n)) * 0.02).astype(np.float32), 4, 64)
+        assert st == 0
+        self.q, self.m, self.a = upload_quantized(kt, q), m, kt.DeviceBuffer.from_numpy(rng.standard_normal((m, n)).astype(np.float32))
+
+    def run(self, stream):
+        self.kt.MatMul.multiply_by_quantized_transposed(self.a, self.q, self.out, self.m, accumulate=False, stream=stream)
+
+
+class _Forward(_Call):
+    def __init__(self, kt, oracle_lib, m, k, n, seed):
+        super().__init__(kt, (m, n))
+        rng = np.random.default_rng(seed)
+        st, q = oracle_lib.quantize((rng.standard_normal((k, n)) * 0.02).astype(np.float32), 4, 64)
+        assert st == 0
+        self.q, self.m, self.a = upload_quantized(kt, q), m, kt.DeviceBuffer.from_numpy(rng.standard_normal((m, k)).astype(np.float32))
+
+    def run(self, stream):
+        self.kt.MatMul.multiply_quantized(self.a, self.q, self.out, self.m, accumulate=False, stream=stream)
+
+
+class _Attention(_Call):
+    def __init__(self, kt, oracle_lib, tokens, heads, kvh, seed):
+        super().__init__(kt, (tokens, heads * 64))
+        rng = np.random.default_rng(seed)
+        self.shape = tokens, heads, kvh
+        self.q, self.k, self.v = (kt.DeviceBuffer.from_numpy(rng.standard_normal((tokens * h * 64,)).astype(np.float32)) for h in (heads, kvh, kvh))
+        self.pos = kt.DeviceBuffer.from_numpy(np.zeros(1, np.int32))
+
+    def run(self, stream):
+        from kotensor_amd import _lib
+        tokens, heads, kvh = self.shape
+        _lib.call("kt_attention", self.q.ptr, tokens, self.pos.ptr, tokens, self.k.ptr, self.v.ptr, 0, tokens, heads, kvh, 64, self.out.ptr,
+                  stream.handle if stream else None)
+
+
+# kind, sizes of the call, sizes of a larger one
+KINDS = [(_Transposed, (64, 1024, 2000), (300, 2048, 4000)), (_Forward, (37, 1000, 2999), (150, 4000, 3001)), (_Attention, (210, 8, 2), (700, 16, 4))]
+IDS = ["transposed", "odd width", "attention"]
+
+
+@contextlib.contextmanager
+def _recorded(call, stream):
+    from kotensor_amd import _lib
+    graph = ctypes.c_void_p()
+    _lib.call("kt_graph_begin", stream.handle)
+    try:
+        call.run(stream)
+    finally:
+        _lib.call("kt_graph_end", stream.handle, ctypes.byref(graph))
+    try:
+        yield graph
+    finally:
+        call.kt.synchronize()
+        _lib.call("kt_graph_destroy", graph)
+
+
+def _replay(call, graph, stream):
+    from kotensor_amd import _lib
+    call.out.fill_zero()
+    call.kt.synchronize()
+    _lib.call("kt_graph_launch", graph, stream.handle)
+    stream.synchronize()
+    return call.result()
+
+
+@pytest.mark.parametrize("kind,sizes,larger", KINDS, ids=IDS)
+@pytest.mark.parametrize("eager_first", [True, False])
+def test_replays_give_the_eager_bits(kt, oracle_lib, kind, sizes, larger, eager_first):
+    """Recorded on a stream with and without eager calls before; a larger eager call on it
+    then replaces its area, and the stream ends before the graph does."""
+    banner("recorded-scratch", kind.__name__, eager_first)
+    call, big = kind(kt, oracle_lib, *sizes, 1), kind(kt, oracle_lib, *larger, 2)
+    want, want_big = call.eager(), big.eager()
+    stream, other = kt.Stream.create(), kt.Stream.create()
+    if eager_first:
+        call.run(stream)
+        stream.synchronize()
+        assert same_bits(call.result(), want)
+    with _recorded(call, stream) as graph:
+        assert same_bits(_replay(call, graph, stream), want)
+        big.run(stream)
+        stream.synchronize()
+        assert same_bits(big.result(), want_big)
+        assert same_bits(_replay(call, graph, stream), want)
+        stream.destroy()
+        for _ in range(2):
+            assert same_bits(_replay(call, graph, other), want)
+            assert same_bits(big.eager(), want_big)
+        other.synchronize()
+    other.destroy()
+
+
+@pytest.mark.parametrize("kind,sizes,larger", KINDS, ids=IDS)
+def test_replays_on_other_streams_do_not_meet(kt, oracle_lib, kind, sizes, larger):
+    """Two graphs recorded on one stream, replayed on two others while that stream runs a
+    third call eagerly: each has the bits it has alone, every time."""
+    from kotensor_amd import _lib
+    banner("recorded-scratch-streams", kind.__name__)
+    calls = [kind(kt, oracle_lib, *sizes, seed) for seed in (1, 2, 3)]
+    want = [c.eager() for c in calls]
+    streams = [kt.Stream.create() for _ in range(3)]
+    calls[2].run(streams[2])
+    streams[2].synchronize()
+    with _recorded(calls[0], streams[2]) as a, _recorded(calls[1], streams[2]) as b:
+        for _ in range(5):
+            for c in calls:
+                c.out.fill_zero()
+            kt.synchronize()
+            for _ in range(20):
+                _lib.call("kt_graph_launch", a, streams[0].handle)
+                _lib.call("kt_graph_launch", b, streams[1].handle)
+                calls[2].run(streams[2])
+            for s in streams:
+                s.synchronize()
+            assert all(same_bits(c.result(), w) for c, w in zip(calls, want))
+    for s in streams:
+        s.destroy()
