@@ -145,8 +145,10 @@ int32_t kt_debug_wait_limits(uint32_t spin_limit, int32_t withhold);
  * kt_attention of 16 and more tokens) may hold scratch of their own: recorded, it belongs
  * to the graph and kt_graph_destroy frees it, so their replays on any stream are
  * independent of eager calls and of other graphs (as for any graph, two replays of one
- * graph write the same outputs and are the caller's to order). A capture begun by other
- * means records them without scratch. */
+ * graph write the same outputs and are the caller's to order). Their results do not depend
+ * on recording or on other threads: the same bits each time, except where there is no
+ * scratch to have (a capture begun by other means, no device memory left); there they run
+ * as single launches whose sums have another order. */
 int32_t kt_graph_begin(void* stream);
 int32_t kt_graph_end(void* stream, void** graph);
 int32_t kt_graph_launch(void* graph, void* stream);

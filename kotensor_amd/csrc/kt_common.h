@@ -67,16 +67,17 @@ WaitLimits wait_limits();
 // not), for calls that have a way to do without its counter region.
 bool workspace_present(hipStream_t stream);
 
-// Scratch that one call holds while it enqueues its launches (two threads on one stream then
-// never interleave launches on it). An eager call takes the area of its stream, which stays for
-// the next call and is freed with the stream; a call recorded between kt_graph_begin and
-// kt_graph_end takes one that belongs to the graph (calls recorded on one stream share it, in
-// stream order) and is freed with it, so that replays on any stream and eager calls never meet
-// in it. ptr stays null where the call does without: more than `limit` bytes, no memory left,
-// another thread's call in progress, a capture begun by other means, whose graph's end the
-// library does not see. (Calls on a caller's fixed workspace get its general area.) The
-// split products' slices and the prefill attention's parts are CALL_SLICES; the fused loss's
-// scratch is CALL_LOSS, since its products want the other.
+// Scratch that one call holds while it enqueues its launches: another thread's call that wants
+// the same area waits until then (they never interleave launches on it). An eager call takes
+// the area of its stream, which stays for the next call and is freed with the stream; a call
+// recorded between kt_graph_begin and kt_graph_end takes one that belongs to the graph (calls
+// recorded on one stream share it, in stream order) and is freed with it, so that replays on any
+// stream and eager calls never meet in it. ptr stays null where there is none to have: no
+// memory left, or a capture begun by other means, whose graph's end the library does not see;
+// what a call takes depends on its shapes alone. (Calls on a caller's fixed workspace get its
+// general area, which holds SLICES_LIMIT bytes.) The split products' slices and the prefill
+// attention's parts are CALL_SLICES; the fused loss's scratch is CALL_LOSS, since its products
+// want the other.
 enum CallArea { CALL_SLICES, CALL_LOSS, CALL_AREAS };
 struct Area {
     void* ptr = nullptr;
@@ -89,13 +90,19 @@ class CallScratch {
     CallScratch(const CallScratch&) = delete;
     CallScratch& operator=(const CallScratch&) = delete;
     ~CallScratch();  // after the call's last launch is enqueued
-    int32_t take(CallArea kind, hipStream_t stream, size_t bytes, size_t limit);
+    int32_t take(CallArea kind, hipStream_t stream, size_t bytes);
     void* ptr = nullptr;
 
   private:
     std::shared_ptr<Area> held_;
 };
-constexpr size_t SLICES_LIMIT = size_t(64) << 20;
+// The fixed device array of kt_qmatmul_noalloc: counters, zeroed accumulators (fp64, half a
+// million columns), then what the split products' slices may take in every call.
+constexpr size_t COUNTER_BYTES = size_t(64) << 10;
+constexpr size_t SCRATCH_BYTES = size_t(64) << 20;
+constexpr size_t SCRATCH_ZERO_BYTES = size_t(4) << 20;
+constexpr size_t SLICES_LIMIT = SCRATCH_BYTES - SCRATCH_ZERO_BYTES - COUNTER_BYTES;
+constexpr size_t PARTS_LIMIT = size_t(64) << 20;
 constexpr size_t LOSS_LIMIT = size_t(192) << 20;
 
 // Validated view of a kt_qweight, with the derived layout numbers.
@@ -162,6 +169,7 @@ int32_t launch_generic(const float* a, int32_t m, const WeightView& w, float* c,
                        float alpha, const float* bias, hipStream_t st);
 int32_t launch_transposed(const float* dy, int32_t m, const WeightView& w, float* dx,
                           int32_t accumulate, hipStream_t st);
+int32_t launch_transposed_rows(const float* dy, int32_t m, const WeightView& w, float* dx, int32_t accumulate, hipStream_t st);
 // Products in fp32 precision on the bf16 matrix units (kt_split.hip): the transposed one and
 // the forward one of any shape and alignment.
 bool forward_split_preferred(int32_t m, const WeightView& w);

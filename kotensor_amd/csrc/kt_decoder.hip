@@ -1114,8 +1114,7 @@ __global__ void __launch_bounds__(THREADS, HD == 64 ? 2 : 1)
 // 8 kv heads of 64 48 -> 42 us; with the call 512 tokens 25 -> 19, 64 after 1024 44 -> 21, 17
 // after 900 40 -> 19; heads of 128 1024 tokens 118 -> 84. Short contexts stay with the tile
 // kernel's one launch (100 tokens, 14 heads: 9.6 against 15 us; 200 of 128 dims 26 against 18),
-// so do calls that get no area for their parts (more than SLICES_LIMIT, a first call under
-// capture, another thread's call in progress).
+// so do calls whose parts exceed PARTS_LIMIT, and those that get no area (CallScratch).
 constexpr int SPLIT_ROWS = 32;
 constexpr int PARTS_MIN_KEYS = 192;
 
@@ -1569,9 +1568,9 @@ static int32_t attention_launch(const float* q, int32_t tokens, const int32_t* p
         a.splits = 1;
         const size_t parts_bytes = static_cast<size_t>(num_kv_heads) * 2 * ceil_div(key_bound, PKT) *
                                    (head_dim == 64 ? parts_block_bytes(64) : parts_block_bytes(128));
-        if (key_bound >= PARTS_MIN_KEYS && G <= SPLIT_ROWS) {
+        if (key_bound >= PARTS_MIN_KEYS && parts_bytes <= PARTS_LIMIT && G <= SPLIT_ROWS) {
             CallScratch parts;
-            if (const int32_t status = parts.take(CALL_SLICES, st, parts_bytes, SLICES_LIMIT)) return status;
+            if (const int32_t status = parts.take(CALL_SLICES, st, parts_bytes)) return status;
             if (parts.ptr)
                 return head_dim == 64 ? launch_prefill_parts<64>(a, tokens, key_bound, static_cast<uint8_t*>(parts.ptr), st)
                                       : launch_prefill_parts<128>(a, tokens, key_bound, static_cast<uint8_t*>(parts.ptr), st);

@@ -223,7 +223,7 @@ extern "C" int32_t kt_fused_cross_entropy(const float* hidden, int32_t rows, con
     CallScratch kept;
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     KT_HIP(hipStreamIsCapturing(st, &capture));
-    if (capture == hipStreamCaptureStatusNone && (status = kept.take(CALL_LOSS, st, bytes, LOSS_LIMIT))) return status;
+    if (capture == hipStreamCaptureStatusNone && bytes <= LOSS_LIMIT && (status = kept.take(CALL_LOSS, st, bytes))) return status;
     void* scratch = kept.ptr;
     if (!kept.ptr) KT_HIP(hipMallocAsync(&scratch, bytes, st));
     float* logits = static_cast<float*>(scratch);

@@ -151,6 +151,10 @@ int32_t launch_generic(const float* a, int32_t m, const WeightView& w, float* c,
 int32_t launch_transposed(const float* dy, int32_t m, const WeightView& w, float* dx, int32_t accumulate,
                           hipStream_t st) {
     if (transposed_split_preferred(m, w)) return launch_transposed_split(dy, m, w, dx, accumulate, st);
+    return launch_transposed_rows(dy, m, w, dx, accumulate, st);
+}
+
+int32_t launch_transposed_rows(const float* dy, int32_t m, const WeightView& w, float* dx, int32_t accumulate, hipStream_t st) {
     dim3 grid;
     int32_t status = grid_1d(static_cast<int64_t>(w.K) * ceil_div(m, TR_ROWS), &grid);
     if (status) return status;

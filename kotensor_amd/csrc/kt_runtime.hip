@@ -4,7 +4,9 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <atomic>
+#include <condition_variable>
 #include <map>
 #include <mutex>
 #include <utility>
@@ -51,6 +53,7 @@ struct Capture {
 };
 std::map<unsigned long long, Capture> g_captures;
 std::map<hipGraphExec_t, std::vector<void*>> g_graph_blocks;
+std::condition_variable g_area_free;  // with g_ws_mutex: a call has enqueued its last launch
 // Blocks replaced or orphaned while a recorded graph may still address them. A graph
 // keeps the addresses it was recorded with, and graphs can outlive their stream, so
 // these stay allocated until the process ends (each is smaller than its successor, so
@@ -75,7 +78,6 @@ thread_local const FixedWorkspace* t_fixed = nullptr;
 // kernel that uses them (the counter region's last words, from ROPE_CACHE_WORD, excepted:
 // the decode attention's RoPE cache, whose entries a zeroed word marks as empty); the
 // general area follows.
-constexpr size_t COUNTER_BYTES = 64 << 10;
 static_assert(ROPE_CACHE_WORD + 512 == COUNTER_BYTES / sizeof(uint32_t), "the RoPE cache ends the counter region");
 
 static int32_t ensure(hipStream_t stream, size_t zbytes, size_t bytes, Block** out) {
@@ -176,9 +178,8 @@ void free_blocks(const std::vector<void*>& blocks) {
 }
 }  // namespace
 
-int32_t CallScratch::take(CallArea kind, hipStream_t stream, size_t bytes, size_t limit) {
-    if (bytes > limit) return KT_OK;
-    if (t_fixed) {  // the fixed workspace's general area, where it is large enough
+int32_t CallScratch::take(CallArea kind, hipStream_t stream, size_t bytes) {
+    if (t_fixed) {
         const size_t head = COUNTER_BYTES + t_fixed->zero_bytes;
         if (bytes <= t_fixed->bytes - head) ptr = t_fixed->ptr + head;
         return KT_OK;
@@ -188,24 +189,29 @@ int32_t CallScratch::take(CallArea kind, hipStream_t stream, size_t bytes, size_
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     unsigned long long id = 0;
     KT_HIP(hipStreamGetCaptureInfo(stream, &status, &id));
-    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    std::unique_lock<std::mutex> lock(g_ws_mutex);
     Capture* capture = nullptr;
-    if (status != hipStreamCaptureStatusNone) {
-        const auto it = g_captures.find(id);
-        if (it == g_captures.end()) return KT_OK;
-        capture = &it->second;
+    std::shared_ptr<Area> area;
+    for (;;) {
+        if (status != hipStreamCaptureStatusNone) {
+            const auto it = g_captures.find(id);
+            if (it == g_captures.end()) return KT_OK;
+            capture = &it->second;
+        }
+        std::shared_ptr<Area>& slot = capture ? capture->areas[std::make_pair(static_cast<int>(kind), stream)]
+                                              : g_areas[kind][std::make_pair(device, stream)];
+        if (!slot) slot = std::make_shared<Area>();
+        area = slot;
+        if (!area->busy) break;
+        g_area_free.wait(lock);  // another thread is enqueuing with it
     }
-    std::shared_ptr<Area>& area = capture ? capture->areas[std::make_pair(static_cast<int>(kind), stream)]
-                                          : g_areas[kind][std::make_pair(device, stream)];
-    if (!area) area = std::make_shared<Area>();
-    if (area->busy) return KT_OK;  // another thread is enqueuing with it
     if (area->bytes < bytes) {
         if (area->ptr && !capture) {
             KT_HIP(hipStreamSynchronize(stream));
             KT_HIP(hipFree(area->ptr));
         }
         *area = Area{};
-        const size_t want = bytes + bytes / 4 < limit ? bytes + bytes / 4 : limit;
+        const size_t want = std::min(bytes + bytes / 4, std::max(bytes, kind == CALL_LOSS ? LOSS_LIMIT : PARTS_LIMIT));
         RelaxedCapture relaxed;
         if (hipMalloc(&area->ptr, want) != hipSuccess) {  // no memory left: the call does without
             (void)hipGetLastError();
@@ -223,8 +229,11 @@ int32_t CallScratch::take(CallArea kind, hipStream_t stream, size_t bytes, size_
 
 CallScratch::~CallScratch() {
     if (!held_) return;
-    std::lock_guard<std::mutex> lock(g_ws_mutex);
-    held_->busy = false;
+    {
+        std::lock_guard<std::mutex> lock(g_ws_mutex);
+        held_->busy = false;
+    }
+    g_area_free.notify_all();
 }
 
 int32_t workspace_counters(hipStream_t stream, size_t bytes, size_t count, void** general, uint32_t** counters) {
@@ -360,8 +369,6 @@ static int32_t check_fault(hipStream_t stream) {
 // process ends). Host code never passes the array's name to a kernel: the name is a
 // host-side stand-in, so each device's address is taken once with hipGetSymbolAddress
 // and kept in g_scratch.
-constexpr size_t SCRATCH_BYTES = 64 << 20;      // counters, accumulators and general area
-constexpr size_t SCRATCH_ZERO_BYTES = 4 << 20;  // fp64 accumulators (half a million columns)
 static __device__ __align__(256) unsigned char scratch[SCRATCH_BYTES];
 
 struct ScratchSlot {

@@ -680,21 +680,13 @@ int32_t launch_slices_reduce(const float* part, int32_t splits, int32_t m, int32
     return KT_OK;
 }
 
-// Slices of `steps` for a grid of `tiles` workgroups: two workgroups per CU, and the area for
-// their sums (slice: bytes of one); one slice, which needs none, where there is no area.
-int32_t choose_slices(hipStream_t st, int64_t tiles, int32_t steps, size_t slice, int32_t* splits, int32_t* per_slice,
-                      CallScratch* area) {
+// Slices of `steps` for a grid of `tiles` workgroups, from the shape alone: two workgroups per
+// CU, as far as the slices' sums (slice: bytes of one) fit SLICES_LIMIT.
+void choose_slices(int64_t tiles, int32_t steps, size_t slice, int32_t* splits, int32_t* per_slice) {
     int64_t want = (2 * cu_count() + tiles - 1) / tiles;
-    want = std::min<int64_t>(std::min<int64_t>(want, MAX_SPLITS), steps);
-    *per_slice = ceil_div(steps, static_cast<int32_t>(want));
+    want = std::min<int64_t>(std::min<int64_t>(want, MAX_SPLITS), std::min<int64_t>(steps, SLICES_LIMIT / slice));
+    *per_slice = ceil_div(steps, static_cast<int32_t>(std::max<int64_t>(want, 1)));
     *splits = ceil_div(steps, *per_slice);
-    if (*splits == 1) return KT_OK;
-    const int32_t status = area->take(CALL_SLICES, st, *splits * slice, SLICES_LIMIT);
-    if (!area->ptr) {
-        *splits = 1;
-        *per_slice = steps;
-    }
-    return status;
 }
 
 template <int BITS, bool ZP, int WM>
@@ -743,9 +735,22 @@ int32_t launch_transposed_split(const float* dy, int32_t m, const WeightView& w,
     const size_t slice = static_cast<size_t>(m) * w.K * sizeof(float);
     const int64_t max_blocks = tiles * MAX_SPLITS;
     if (max_blocks > INT32_MAX) return fail(KT_ERR_SHAPE, "grid of %lld blocks is out of range", static_cast<long long>(max_blocks));
+    choose_slices(tiles, p.steps, slice, &p.splits, &p.steps_per_split);
     CallScratch area;
-    if (const int32_t status = choose_slices(st, tiles, p.steps, slice, &p.splits, &p.steps_per_split, &area)) return status;
-    if (area.ptr) p.out = static_cast<float*>(area.ptr);
+    if (p.splits > 1) {
+        if (const int32_t status = area.take(CALL_SLICES, st, p.splits * slice)) return status;
+        if (area.ptr) {
+            p.out = static_cast<float*>(area.ptr);
+        } else {
+            // No scratch to have (CallScratch): one slice, or the row-by-row kernel where the few
+            // workgroups of one slice would take longer. Row by row / one slice, 2048 -> 8192:
+            // M = 1 28 / 460 us, 32 225 / 479, 48 334 / 362, 64 446 / 394, 512 2822 / 361; M = 200
+            // 640 -> 100 30 / 19, M = 8 9000 -> 2000 60 / 129.
+            if (int64_t{ceil_div(m, 8)} * w.K * w.N < int64_t{p.steps} * (7 << 17)) return launch_transposed_rows(dy, m, w, dx, accumulate, st);
+            p.splits = 1;
+            p.steps_per_split = p.steps;
+        }
+    }
     // Runs: no longer a sequence of sums than the row-by-row kernel's N / 256, or 16 steps
     // (28 steps in one run at N = 3584 had 1.19e-7 of the 2-norm against its 1.04e-7, two
     // runs of 14 have 1.01e-7; each run after a slice's first takes about 7 us).
@@ -784,9 +789,17 @@ int32_t launch_forward_split(const float* a, int32_t m, const WeightView& w, flo
     const size_t slice = static_cast<size_t>(m) * w.N * sizeof(float);
     const int64_t max_blocks = tiles * MAX_SPLITS;
     if (max_blocks > INT32_MAX) return fail(KT_ERR_SHAPE, "grid of %lld blocks is out of range", static_cast<long long>(max_blocks));
+    choose_slices(tiles, p.steps, slice, &p.splits, &p.steps_per_split);
     CallScratch area;
-    if (const int32_t status = choose_slices(st, tiles, p.steps, slice, &p.splits, &p.steps_per_split, &area)) return status;
-    if (area.ptr) p.c = static_cast<float*>(area.ptr);
+    if (p.splits > 1) {
+        if (const int32_t status = area.take(CALL_SLICES, st, p.splits * slice)) return status;
+        if (area.ptr) {
+            p.c = static_cast<float*>(area.ptr);
+        } else {  // no scratch to have (CallScratch): one slice (3 us a step of 64 k; generic_matmul 9)
+            p.splits = 1;
+            p.steps_per_split = p.steps;
+        }
+    }
     const uint32_t blocks = static_cast<uint32_t>(tiles * p.splits);
     if (w.bits == 4) launch_forward_rows<4, true>(wm, p, blocks, st);
     else if (w.z) launch_forward_rows<8, true>(wm, p, blocks, st);

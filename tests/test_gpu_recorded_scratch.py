@@ -149,3 +149,80 @@ def test_replays_on_other_streams_do_not_meet(kt, oracle_lib, kind, sizes, large
             assert all(same_bits(c.result(), w) for c, w in zip(calls, want))
     for s in streams:
         s.destroy()
+
+
+@pytest.mark.parametrize("kind,sizes", [(_Transposed, (16, 1024, 4000)), (_Transposed, (200, 640, 1000)), (_Forward, (37, 1000, 2999)), (_Attention, (210, 8, 2))])
+def test_a_callers_own_capture(kt, oracle_lib, kind, sizes):
+    """A capture begun with HIP itself records the forms without scratch: the row-by-row
+    kernel (16 rows) or one slice, the attention kernel that splits tiles itself. Their sums
+    have another order: 1e-6 normwise, the bound of the products' and the attention's tests."""
+    banner("recorded-scratch-own-capture", kind.__name__, *sizes)
+    call = kind(kt, oracle_lib, *sizes, 4)
+    want = call.eager()
+    with open("/proc/self/maps") as maps:
+        hip = ctypes.CDLL(next(line.split()[-1] for line in maps if "libamdhip64" in line))
+    stream, graph, exe = kt.Stream.create(), ctypes.c_void_p(), ctypes.c_void_p()
+    call.run(stream)  # an area that the recorded call must not take
+    stream.synchronize()
+    handle = ctypes.c_void_p(stream.handle)
+    assert hip.hipStreamBeginCapture(handle, 1) == 0  # thread-local
+    try:
+        call.run(stream)
+    finally:
+        assert hip.hipStreamEndCapture(handle, ctypes.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, ctypes.c_size_t(0)) == 0
+    assert hip.hipGraphDestroy(graph) == 0
+    for _ in range(3):
+        got = _replay(call, exe, stream)
+        assert np.linalg.norm(got.astype(np.float64) - want) <= 1e-6 * np.linalg.norm(want)
+        assert same_bits(call.eager(), want)
+    assert hip.hipGraphExecDestroy(exe) == 0
+    stream.destroy()
+
+
+@pytest.mark.parametrize("kind,sizes,larger", KINDS, ids=IDS)
+def test_two_threads_give_the_same_bits(kt, oracle_lib, kind, sizes, larger):
+    """Two threads call on the null stream at once: each result has the bits it has alone."""
+    import threading
+
+    banner("scratch-two-threads", kind.__name__)
+    calls = [[kind(kt, oracle_lib, *s, 10 * i + j) for j, s in enumerate((sizes, larger))] for i in range(2)]
+    want = [[c.eager() for c in pair] for pair in calls]
+    bad = []
+
+    def work(i):
+        for _ in range(20):
+            for c in calls[i]:
+                c.run(None)
+        kt.synchronize()
+        bad.extend(not same_bits(c.result(), w) for c, w in zip(calls[i], want[i]))
+
+    for pair in calls:
+        for c in pair:
+            c.out.fill_zero()
+    kt.synchronize()
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(bad) == 4 and not any(bad)
+
+
+# slices of every size: many, few, and (2560 rows) two that would need 62.5 MiB, more than the
+# fixed array's general area
+@pytest.mark.parametrize("m,k,n,bits", [(1, 4096, 1023, 4), (37, 1000, 2999, 4), (200, 2000, 515, 8), (2560, 256, 3199, 4)])
+def test_noalloc_gives_the_bits_of_the_plain_product(kt, oracle_lib, m, k, n, bits):
+    from kotensor_amd import _lib
+    banner("scratch-noalloc", m, k, n, bits)
+    rng = np.random.default_rng(m)
+    st, q = oracle_lib.quantize((rng.standard_normal((k, n)) * 0.02).astype(np.float32), bits, 64)
+    assert st == 0
+    qt, a = upload_quantized(kt, q), kt.DeviceBuffer.from_numpy(rng.standard_normal((m, k)).astype(np.float32))
+    got = []
+    for entry in ("kt_qmatmul", "kt_qmatmul_noalloc"):
+        c = kt.DeviceBuffer(m * n * 4)
+        _lib.call(entry, a.ptr, m, ctypes.byref(qt.qweight), c.ptr, 0, ctypes.c_float(1.0), None)
+        kt.synchronize()
+        got.append(c.download(np.float32))
+    assert same_bits(*got)
