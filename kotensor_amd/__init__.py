@@ -11,7 +11,7 @@ device-resident decoder around the projections (``Transformer``, ``KVCache``,
 quantized head (``fused_cross_entropy_loss``).
 """
 from ._lib import IllegalArgumentException, IllegalStateException, LibraryMissingError, LIBRARY_PATH
-from .device import DeviceBuffer, Stream, synchronize, device_count
+from .device import DeviceBuffer, Stream, synchronize, device_count, release_scratch
 from .quantization import Quantization, QuantizedTensor
 from .matmul import MatMul, DeviceTensor
 from .linear import QuantizedLinear, projection, forward_into_group
@@ -28,6 +28,7 @@ __all__ = [
     "Stream",
     "synchronize",
     "device_count",
+    "release_scratch",
     "Quantization",
     "QuantizedTensor",
     "MatMul",

@@ -67,18 +67,25 @@ WaitLimits wait_limits();
 // not), for calls that have a way to do without its counter region.
 bool workspace_present(hipStream_t stream);
 
-// Scratch that one call holds while it enqueues its launches: another thread's call that wants
-// the same area waits until then (they never interleave launches on it). An eager call takes
-// the area of its stream, which stays for the next call and is freed with the stream; a call
-// recorded between kt_graph_begin and kt_graph_end takes one that belongs to the graph (calls
-// recorded on one stream share it, in stream order) and is freed with it, so that replays on any
-// stream and eager calls never meet in it. ptr stays null where there is none to have: no
+// Scratch of one call, held until it has enqueued its launches. Device memory is from a pool of
+// the library's per device, in stream order: no call waits for a stream to get or grow it, and
+// at most POOL_KEPT bytes stay in the pool when nothing uses them (scratch_release and
+// kt_stream_destroy give them back).
+//
+// take: an area that stays for the next call (the split products' slices, the prefill
+// attention's parts; getting memory from the pool for each call costs 10 us of host time).
+// Another thread's call that wants the same area waits until this one has enqueued its
+// launches, so they never interleave on it. An eager call takes the area of its stream; a
+// call recorded between kt_graph_begin and kt_graph_end takes one that belongs to the graph
+// (calls recorded on one stream share it, in stream order) and is freed with it, so that
+// replays on any stream and eager calls never meet in it. hipStreamPerThread, one handle for
+// many streams, has no area: its calls allocate. ptr stays null where there is none to have: no
 // memory left, or a capture begun by other means, whose graph's end the library does not see;
 // what a call takes depends on its shapes alone. (Calls on a caller's fixed workspace get its
-// general area, which holds SLICES_LIMIT bytes.) The split products' slices and the prefill
-// attention's parts are CALL_SLICES; the fused loss's scratch is CALL_LOSS, since its products
-// want the other.
-enum CallArea { CALL_SLICES, CALL_LOSS, CALL_AREAS };
+// general area, which holds SLICES_LIMIT bytes.)
+//
+// allocate: memory for this call only, freed on the stream behind its launches (the fused
+// loss); ptr stays null if there is none left. In a capture it becomes part of the graph.
 struct Area {
     void* ptr = nullptr;
     size_t bytes = 0;
@@ -90,12 +97,19 @@ class CallScratch {
     CallScratch(const CallScratch&) = delete;
     CallScratch& operator=(const CallScratch&) = delete;
     ~CallScratch();  // after the call's last launch is enqueued
-    int32_t take(CallArea kind, hipStream_t stream, size_t bytes);
+    int32_t take(hipStream_t stream, size_t bytes);
+    int32_t allocate(hipStream_t stream, size_t bytes);
     void* ptr = nullptr;
 
   private:
     std::shared_ptr<Area> held_;
+    bool allocated_ = false;
+    hipStream_t stream_ = nullptr;
 };
+// Waits for the device and gives back every area that no call is enqueuing with, then the
+// pool's unused memory.
+int32_t scratch_release();
+constexpr uint64_t POOL_KEPT = uint64_t(256) << 20;
 // The fixed device array of kt_qmatmul_noalloc: counters, zeroed accumulators (fp64, half a
 // million columns), then what the split products' slices may take in every call.
 constexpr size_t COUNTER_BYTES = size_t(64) << 10;
@@ -103,7 +117,6 @@ constexpr size_t SCRATCH_BYTES = size_t(64) << 20;
 constexpr size_t SCRATCH_ZERO_BYTES = size_t(4) << 20;
 constexpr size_t SLICES_LIMIT = SCRATCH_BYTES - SCRATCH_ZERO_BYTES - COUNTER_BYTES;
 constexpr size_t PARTS_LIMIT = size_t(64) << 20;
-constexpr size_t LOSS_LIMIT = size_t(192) << 20;
 
 // Validated view of a kt_qweight, with the derived layout numbers.
 struct WeightView {

@@ -218,64 +218,53 @@ extern "C" int32_t kt_fused_cross_entropy(const float* hidden, int32_t rows, con
     const size_t logit_bytes = static_cast<size_t>(pass) * V * sizeof(float);
     const size_t row_bytes = static_cast<size_t>(pass) * K * sizeof(float);
     const size_t bytes = logit_bytes + 2 * row_bytes + static_cast<size_t>(active) * (sizeof(float) + 2 * sizeof(int32_t));
-    // the stream's kept area; an allocation of this call where there is none (67 MB allocated
-    // and freed on every call cost 50 to 250 us)
-    CallScratch kept;
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    KT_HIP(hipStreamIsCapturing(st, &capture));
-    if (capture == hipStreamCaptureStatusNone && bytes <= LOSS_LIMIT && (status = kept.take(CALL_LOSS, st, bytes))) return status;
-    void* scratch = kept.ptr;
-    if (!kept.ptr) KT_HIP(hipMallocAsync(&scratch, bytes, st));
+    CallScratch area;
+    if ((status = area.allocate(st, bytes))) return status;
+    if (!area.ptr) return hip_fail(hipErrorOutOfMemory, "fused cross-entropy: scratch");
+    void* scratch = area.ptr;
     float* logits = static_cast<float*>(scratch);
     float* inputs = reinterpret_cast<float*>(static_cast<char*>(scratch) + logit_bytes);
     float* pass_grad = reinterpret_cast<float*>(static_cast<char*>(scratch) + logit_bytes + row_bytes);
     float* row_loss = reinterpret_cast<float*>(static_cast<char*>(scratch) + logit_bytes + 2 * row_bytes);
     int32_t* drows = reinterpret_cast<int32_t*>(row_loss + active);
     int32_t* dtargets = drows + active;
-    status = [&]() -> int32_t {
-        // pageable source: the copy has read it when the call returns
-        KT_HIP(hipMemcpyAsync(drows, act.data(), act.size() * sizeof(int32_t), hipMemcpyHostToDevice, st));
-        if (hidden_grad && !accumulate) {  // ignored rows' gradient is zero
-            const int32_t f = fill(hidden_grad, static_cast<int64_t>(rows) * K, 0.0f, st);
-            if (f) return f;
+    // pageable source: the copy has read it when the call returns
+    KT_HIP(hipMemcpyAsync(drows, act.data(), act.size() * sizeof(int32_t), hipMemcpyHostToDevice, st));
+    if (hidden_grad && !accumulate) {  // ignored rows' gradient is zero
+        const int32_t f = fill(hidden_grad, static_cast<int64_t>(rows) * K, 0.0f, st);
+        if (f) return f;
+    }
+    const float scale = 1.0f / static_cast<float>(active);
+    for (int32_t start = 0; start < active; start += pass) {
+        const int32_t count = std::min(pass, active - start);
+        gather_rows_kernel<<<count, 256, 0, st>>>(hidden, K, drows + start, inputs);
+        KT_LAUNCHED("fused cross-entropy: gather rows");
+        // The chunks' products. Chunks of more than 16 rows go through the same kernel
+        // row by row, so they make one product (a shorter last chunk its own).
+        int32_t s = KT_OK;
+        for (int32_t c = 0; c < count && s == KT_OK;) {
+            const int32_t left = count - c;
+            const int32_t n = chunk <= 16 ? std::min(chunk, left) : left % chunk > 16 ? left : left < chunk ? left : left - left % chunk;
+            s = qmatmul(inputs + static_cast<int64_t>(c) * K, n, head, logits + static_cast<int64_t>(c) * V, 0, 1.0f, bias, st);
+            c += n;
         }
-        const float scale = 1.0f / static_cast<float>(active);
-        for (int32_t start = 0; start < active; start += pass) {
-            const int32_t count = std::min(pass, active - start);
-            gather_rows_kernel<<<count, 256, 0, st>>>(hidden, K, drows + start, inputs);
-            KT_LAUNCHED("fused cross-entropy: gather rows");
-            // The chunks' products. Chunks of more than 16 rows go through the same kernel
-            // row by row, so they make one product (a shorter last chunk its own).
-            int32_t s = KT_OK;
-            for (int32_t c = 0; c < count && s == KT_OK;) {
-                const int32_t left = count - c;
-                const int32_t n = chunk <= 16 ? std::min(chunk, left) : left % chunk > 16 ? left : left < chunk ? left : left - left % chunk;
-                s = qmatmul(inputs + static_cast<int64_t>(c) * K, n, head, logits + static_cast<int64_t>(c) * V, 0, 1.0f, bias, st);
-                c += n;
-            }
+        if (s) return s;
+        ce_rows_kernel<<<count, CE_THREADS, 0, st>>>(logits, V, dtargets + start, scale, row_loss + start,
+                                                     grads ? 1 : 0);
+        KT_LAUNCHED("fused cross-entropy: rows");
+        if (bias_grad) {
+            ce_bias_grad_kernel<<<ceil_div(V, 64), 64 * BIAS_WAVES, 0, st>>>(logits, count, V, bias_grad,
+                                                                          (accumulate || start > 0) ? 1 : 0);
+            KT_LAUNCHED("fused cross-entropy: bias gradient");
+        }
+        if (hidden_grad) {
+            s = launch_transposed(logits, count, w, pass_grad, 0, st);
             if (s) return s;
-            ce_rows_kernel<<<count, CE_THREADS, 0, st>>>(logits, V, dtargets + start, scale, row_loss + start,
-                                                         grads ? 1 : 0);
-            KT_LAUNCHED("fused cross-entropy: rows");
-            if (bias_grad) {
-                ce_bias_grad_kernel<<<ceil_div(V, 64), 64 * BIAS_WAVES, 0, st>>>(logits, count, V, bias_grad,
-                                                                              (accumulate || start > 0) ? 1 : 0);
-                KT_LAUNCHED("fused cross-entropy: bias gradient");
-            }
-            if (hidden_grad) {
-                s = launch_transposed(logits, count, w, pass_grad, 0, st);
-                if (s) return s;
-                scatter_rows_kernel<<<count, 256, 0, st>>>(pass_grad, K, drows + start, hidden_grad, accumulate);
-                KT_LAUNCHED("fused cross-entropy: scatter rows");
-            }
+            scatter_rows_kernel<<<count, 256, 0, st>>>(pass_grad, K, drows + start, hidden_grad, accumulate);
+            KT_LAUNCHED("fused cross-entropy: scatter rows");
         }
-        ce_loss_kernel<<<1, CE_THREADS, 0, st>>>(row_loss, active, active, loss);
-        KT_LAUNCHED("fused cross-entropy: loss");
-        return KT_OK;
-    }();
-    hipError_t freed = hipSuccess;
-    if (!kept.ptr) freed = hipFreeAsync(scratch, st);
-    if (status) return status;
-    if (freed != hipSuccess) return hip_fail(freed, "hipFreeAsync");
+    }
+    ce_loss_kernel<<<1, CE_THREADS, 0, st>>>(row_loss, active, active, loss);
+    KT_LAUNCHED("fused cross-entropy: loss");
     return KT_OK;
 }

@@ -42,14 +42,14 @@ struct Block {
 };
 std::mutex g_ws_mutex;
 std::map<std::pair<int, hipStream_t>, Block> g_ws;
-// The areas of the streams' eager calls, per kind (CallScratch).
-std::map<std::pair<int, hipStream_t>, std::shared_ptr<Area>> g_areas[CALL_AREAS];
+// The areas of the streams' eager calls (CallScratch), from g_pools.
+std::map<std::pair<int, hipStream_t>, std::shared_ptr<Area>> g_areas;
 // The areas of recorded calls, while their capture runs (by its id) and once it is a graph:
 // the graph's end frees them.
 struct Capture {
-    hipStream_t origin = nullptr;                          // the stream of kt_graph_begin
-    std::map<std::pair<int, hipStream_t>, std::shared_ptr<Area>> areas;  // by kind and stream
-    std::vector<void*> blocks;                             // all that the recorded calls may address
+    hipStream_t origin = nullptr;  // the stream of kt_graph_begin
+    std::map<hipStream_t, std::shared_ptr<Area>> areas;
+    std::vector<void*> blocks;     // all that the recorded calls may address
 };
 std::map<unsigned long long, Capture> g_captures;
 std::map<hipGraphExec_t, std::vector<void*>> g_graph_blocks;
@@ -61,6 +61,7 @@ std::condition_variable g_area_free;  // with g_ws_mutex: a call has enqueued it
 std::vector<void*> g_retired;
 constexpr int MAX_DEVICES = 64;
 int32_t g_cus[MAX_DEVICES] = {};  // compute units per device, 0 until asked
+hipMemPool_t g_pools[MAX_DEVICES] = {};  // each device's pool of scratch memory, once one is needed
 
 // A caller-provided workspace that replaces the per-stream one for the calls this
 // thread makes while it is set (kt_qmatmul_noalloc), laid out like a stream's:
@@ -178,7 +179,39 @@ void free_blocks(const std::vector<void*>& blocks) {
 }
 }  // namespace
 
-int32_t CallScratch::take(CallArea kind, hipStream_t stream, size_t bytes) {
+namespace {
+// `bytes` of the device's pool, in stream order; *out is null if there is no memory left.
+// With g_ws_mutex held.
+int32_t pool_alloc(int device, hipStream_t stream, size_t bytes, void** out) {
+    *out = nullptr;
+    if (device < 0 || device >= MAX_DEVICES) return fail(KT_ERR_ARGUMENT, "device %d out of range", device);
+    hipMemPool_t& pool = g_pools[device];
+    if (!pool) {
+        hipMemPoolProps props{};
+        props.allocType = hipMemAllocationTypePinned;
+        props.location.type = hipMemLocationTypeDevice;
+        props.location.id = device;
+        KT_HIP(hipMemPoolCreate(&pool, &props));
+        uint64_t kept = POOL_KEPT;
+        KT_HIP(hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &kept));
+    }
+    const hipError_t err = hipMallocFromPoolAsync(out, bytes, pool, stream);
+    if (err == hipSuccess) return KT_OK;
+    *out = nullptr;
+    (void)hipGetLastError();
+    return err == hipErrorOutOfMemory ? KT_OK : hip_fail(err, "hipMallocFromPoolAsync");
+}
+
+// Gives the pool's unused memory of the current device back.
+void pool_trim() {
+    int device = 0;
+    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= MAX_DEVICES) return;
+    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    if (g_pools[device]) (void)hipMemPoolTrimTo(g_pools[device], 0);
+}
+}  // namespace
+
+int32_t CallScratch::take(hipStream_t stream, size_t bytes) {
     if (t_fixed) {
         const size_t head = COUNTER_BYTES + t_fixed->zero_bytes;
         if (bytes <= t_fixed->bytes - head) ptr = t_fixed->ptr + head;
@@ -189,6 +222,7 @@ int32_t CallScratch::take(CallArea kind, hipStream_t stream, size_t bytes) {
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     unsigned long long id = 0;
     KT_HIP(hipStreamGetCaptureInfo(stream, &status, &id));
+    if (status == hipStreamCaptureStatusNone && stream == hipStreamPerThread) return allocate(stream, bytes);
     std::unique_lock<std::mutex> lock(g_ws_mutex);
     Capture* capture = nullptr;
     std::shared_ptr<Area> area;
@@ -198,27 +232,30 @@ int32_t CallScratch::take(CallArea kind, hipStream_t stream, size_t bytes) {
             if (it == g_captures.end()) return KT_OK;
             capture = &it->second;
         }
-        std::shared_ptr<Area>& slot = capture ? capture->areas[std::make_pair(static_cast<int>(kind), stream)]
-                                              : g_areas[kind][std::make_pair(device, stream)];
+        std::shared_ptr<Area>& slot = capture ? capture->areas[stream] : g_areas[std::make_pair(device, stream)];
         if (!slot) slot = std::make_shared<Area>();
         area = slot;
         if (!area->busy) break;
         g_area_free.wait(lock);  // another thread is enqueuing with it
     }
     if (area->bytes < bytes) {
-        if (area->ptr && !capture) {
-            KT_HIP(hipStreamSynchronize(stream));
-            KT_HIP(hipFree(area->ptr));
+        const size_t want = std::min(bytes + bytes / 4, std::max(bytes, PARTS_LIMIT));
+        if (capture) {  // a smaller block stays with the graph, whose earlier calls use it
+            *area = Area{};
+            RelaxedCapture relaxed;
+            if (hipMalloc(&area->ptr, want) != hipSuccess) {
+                (void)hipGetLastError();
+                area->ptr = nullptr;
+                return KT_OK;
+            }
+            capture->blocks.push_back(area->ptr);
+        } else {
+            void* old = area->ptr;
+            *area = Area{};
+            if (old) KT_HIP(hipFreeAsync(old, stream));  // behind the calls that use it
+            const int32_t s = pool_alloc(device, stream, want, &area->ptr);
+            if (s || !area->ptr) return s;
         }
-        *area = Area{};
-        const size_t want = std::min(bytes + bytes / 4, std::max(bytes, kind == CALL_LOSS ? LOSS_LIMIT : PARTS_LIMIT));
-        RelaxedCapture relaxed;
-        if (hipMalloc(&area->ptr, want) != hipSuccess) {  // no memory left: the call does without
-            (void)hipGetLastError();
-            area->ptr = nullptr;
-            return KT_OK;
-        }
-        if (capture) capture->blocks.push_back(area->ptr);
         area->bytes = want;
     }
     area->busy = true;
@@ -227,13 +264,50 @@ int32_t CallScratch::take(CallArea kind, hipStream_t stream, size_t bytes) {
     return KT_OK;
 }
 
+int32_t CallScratch::allocate(hipStream_t stream, size_t bytes) {
+    int device = 0;
+    KT_HIP(hipGetDevice(&device));
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    KT_HIP(hipStreamIsCapturing(stream, &capture));
+    if (capture != hipStreamCaptureStatusNone) {
+        KT_HIP(hipMallocAsync(&ptr, bytes, stream));
+    } else {
+        std::lock_guard<std::mutex> lock(g_ws_mutex);
+        if (const int32_t s = pool_alloc(device, stream, bytes, &ptr)) return s;
+    }
+    allocated_ = ptr != nullptr;
+    stream_ = stream;
+    return KT_OK;
+}
+
 CallScratch::~CallScratch() {
+    if (allocated_ && hipFreeAsync(ptr, stream_) != hipSuccess) (void)hipGetLastError();
     if (!held_) return;
     {
         std::lock_guard<std::mutex> lock(g_ws_mutex);
         held_->busy = false;
     }
     g_area_free.notify_all();
+}
+
+int32_t scratch_release() {
+    int device = 0;
+    KT_HIP(hipGetDevice(&device));
+    {
+        std::lock_guard<std::mutex> lock(g_ws_mutex);
+        KT_HIP(hipDeviceSynchronize());
+        for (auto it = g_areas.begin(); it != g_areas.end();) {
+            if (it->first.first != device || it->second->busy) {
+                ++it;
+                continue;
+            }
+            if (it->second->ptr) KT_HIP(hipFreeAsync(it->second->ptr, nullptr));
+            it = g_areas.erase(it);
+        }
+    }
+    KT_HIP(hipStreamSynchronize(nullptr));
+    pool_trim();
+    return KT_OK;
 }
 
 int32_t workspace_counters(hipStream_t stream, size_t bytes, size_t count, void** general, uint32_t** counters) {
@@ -491,7 +565,13 @@ int32_t kt_dev_alloc(size_t bytes, void** ptr) {
     if (!ptr) return fail(KT_ERR_ARGUMENT, "ptr is NULL");
     *ptr = nullptr;
     if (bytes == 0) return KT_OK;
-    KT_HIP(hipMalloc(ptr, bytes));
+    hipError_t err = hipMalloc(ptr, bytes);
+    if (err == hipErrorOutOfMemory) {  // once more without what the scratch pool keeps
+        (void)hipGetLastError();
+        pool_trim();
+        err = hipMalloc(ptr, bytes);
+    }
+    if (err != hipSuccess) return hip_fail(err, "hipMalloc(ptr, bytes)");
     return KT_OK;
 }
 
@@ -544,7 +624,7 @@ int32_t kt_stream_create(void** stream) {
 }
 
 int32_t kt_stream_destroy(void* stream) {
-    if (!stream) return KT_OK;
+    if (!stream) return scratch_release();
     hipStream_t s = static_cast<hipStream_t>(stream);
     KT_HIP(hipStreamSynchronize(s));
     {
@@ -558,13 +638,14 @@ int32_t kt_stream_destroy(void* stream) {
             else if (it->second.ptr) KT_HIP(hipFree(it->second.ptr));
             g_ws.erase(it);
         }
-        for (auto& areas : g_areas) {
-            const auto area = areas.find(std::make_pair(device, s));
-            if (area == areas.end()) continue;
-            if (area->second->ptr) KT_HIP(hipFree(area->second->ptr));
-            areas.erase(area);
+        const auto area = g_areas.find(std::make_pair(device, s));
+        if (area != g_areas.end()) {
+            if (area->second->ptr) KT_HIP(hipFreeAsync(area->second->ptr, s));
+            g_areas.erase(area);
         }
     }
+    KT_HIP(hipStreamSynchronize(s));
+    pool_trim();
     KT_HIP(hipStreamDestroy(s));
     return KT_OK;
 }

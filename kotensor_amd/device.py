@@ -119,6 +119,11 @@ def synchronize(stream: Stream | None = None) -> None:
     (stream or _NULL).synchronize()
 
 
+def release_scratch() -> None:
+    """Waits for the device and gives back the scratch memory the library keeps between calls."""
+    _lib.call("kt_stream_destroy", None)
+
+
 def device_count() -> int:
     n = ctypes.c_int32()
     _lib.call("kt_device_count", ctypes.byref(n))

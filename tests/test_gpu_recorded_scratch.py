@@ -72,6 +72,12 @@ KINDS = [(_Transposed, (64, 1024, 2000), (300, 2048, 4000)), (_Forward, (37, 100
 IDS = ["transposed", "odd width", "attention"]
 
 
+def _hip():
+    """The HIP runtime that the library loaded."""
+    with open("/proc/self/maps") as maps:
+        return ctypes.CDLL(next(line.split()[-1] for line in maps if "libamdhip64" in line))
+
+
 @contextlib.contextmanager
 def _recorded(call, stream):
     from kotensor_amd import _lib
@@ -159,8 +165,7 @@ def test_a_callers_own_capture(kt, oracle_lib, kind, sizes):
     banner("recorded-scratch-own-capture", kind.__name__, *sizes)
     call = kind(kt, oracle_lib, *sizes, 4)
     want = call.eager()
-    with open("/proc/self/maps") as maps:
-        hip = ctypes.CDLL(next(line.split()[-1] for line in maps if "libamdhip64" in line))
+    hip = _hip()
     stream, graph, exe = kt.Stream.create(), ctypes.c_void_p(), ctypes.c_void_p()
     call.run(stream)  # an area that the recorded call must not take
     stream.synchronize()
@@ -226,3 +231,70 @@ def test_noalloc_gives_the_bits_of_the_plain_product(kt, oracle_lib, m, k, n, bi
         kt.synchronize()
         got.append(c.download(np.float32))
     assert same_bits(*got)
+
+
+def _free_bytes():
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert _hip().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_scratch_is_given_back(kt, oracle_lib):
+    """What calls kept on the null stream, on a stream of the library and on one that its
+    owner destroyed, and what graphs had: free again after release_scratch and the graphs'
+    ends (within 8 MiB for what the runtime itself keeps; a call here keeps 40 MB)."""
+    banner("scratch-given-back")
+    call = _Transposed(kt, oracle_lib, 512, 2048, 4096, 5)
+    call.eager()
+    kt.release_scratch()
+    before = _free_bytes()
+    call.eager()
+    assert _free_bytes() < before - (32 << 20)
+    own, theirs = kt.Stream.create(), ctypes.c_void_p()
+    hip = _hip()
+    assert hip.hipStreamCreate(ctypes.byref(theirs)) == 0
+    for s in (own, kt.Stream(theirs.value)):
+        call.run(s)
+        s.synchronize()
+    own.destroy()
+    assert hip.hipStreamDestroy(theirs) == 0
+    want = call.eager()
+    stream = kt.Stream.create()
+    for _ in range(10):  # 40 MB a graph
+        with _recorded(call, stream) as graph:
+            assert same_bits(_replay(call, graph, stream), want)
+    stream.destroy()
+    kt.release_scratch()
+    assert _free_bytes() > before - (8 << 20)
+    assert same_bits(call.eager(), want)
+
+
+@pytest.mark.parametrize("kind,sizes,larger", KINDS, ids=IDS)
+def test_the_per_thread_stream(kt, oracle_lib, kind, sizes, larger):
+    """hipStreamPerThread is one handle for a stream of each thread: two threads' calls on it
+    run at once and keep their bits."""
+    import threading
+
+    banner("scratch-per-thread-stream", kind.__name__)
+    calls = [[kind(kt, oracle_lib, *s, 10 * i + j) for j, s in enumerate((sizes, larger))] for i in range(2)]
+    want = [[c.eager() for c in pair] for pair in calls]
+    for pair in calls:
+        for c in pair:
+            c.out.fill_zero()
+    kt.synchronize()
+    bad = []
+
+    def work(i):
+        stream = kt.Stream(2)
+        for _ in range(20):
+            for c in calls[i]:
+                c.run(stream)
+        stream.synchronize()
+        bad.extend(not same_bits(c.result(), w) for c, w in zip(calls[i], want[i]))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(bad) == 4 and not any(bad)
