@@ -823,10 +823,11 @@ __global__ void __launch_bounds__(64 * DIRECT_WAVES) attention_direct_kernel(Att
 // r = (token t0 + r / G, head g G + r % G), r < 64, over keys 0 .. position + token, 64 keys
 // at a time. Wave w takes rows 32 (w % 2) .. + 31 and keys 32 (w / 2) .. + 31 of every tile;
 // the two key halves of a row meet at the end, through LDS.
-// An fp32 number is the exact sum of three bf16 numbers (kt_split.h); the product of two is
-// taken as the six products of parts down to 2^-16 of the largest (the three left out are
-// below an fp32 rounding), on v_mfma_f32_32x32x16_bf16 with fp32 sums, small products first:
-// 2.7 times the rate of the fp32 matrix instruction.
+// An fp32 number is the exact sum of three bf16 numbers, each the nearest to what is left
+// (split3_nearest, kt_split.h); the product of two is taken as the six products of parts down to
+// 2^-17 of the largest (the three left out come to at most 2^-24 of the product, an fp32
+// rounding, and are as often above as below), on v_mfma_f32_32x32x16_bf16 with fp32 sums, small
+// products first: 2.7 times the rate of the fp32 matrix instruction.
 //   S^T = K Q^T: lane l ends with the scores of query row l % 32 against the 16 keys
 //     8 (e / 4) + 4 (l / 32) + e % 4 of the wave's 32 (register e), so the running maximum,
 //     the exponentials and the rescaling of a row stay inside lanes l, l ^ 32. Q is scaled
@@ -922,7 +923,7 @@ __global__ void __launch_bounds__(THREADS, HD == 64 ? 2 : 1)
             v[e] = v0[e] * qscale;
             v[4 + e] = v1[e] * qscale;
         }
-        split3(v, qp[s]);
+        split3_nearest(v, qp[s]);
     }
     // rows of the wave: the first and last key any of them sees last
     int32_t p_min = row_ok ? p_r : 0x7FFFFFFF, p_max = p_r;
@@ -961,11 +962,11 @@ __global__ void __launch_bounds__(THREADS, HD == 64 ? 2 : 1)
         for (int i = 0; i < NI; ++i) {
             const int32_t e = tid + i * THREADS;
             bf16x8 part[3];
-            split3(kr[i], part);
+            split3_nearest(kr[i], part);
 #pragma unroll
             for (int h = 0; h < 3; ++h)
                 *reinterpret_cast<bf16x8*>(&sh.k[h][e / (HD / 8)][8 * (e % (HD / 8))]) = part[h];
-            split3(vr[i], part);
+            split3_nearest(vr[i], part);
 #pragma unroll
             for (int h = 0; h < 3; ++h) *reinterpret_cast<bf16x8*>(&sh.v[h][e % HD][8 * (e / HD)]) = part[h];
         }
@@ -1022,7 +1023,7 @@ __global__ void __launch_bounds__(THREADS, HD == 64 ? 2 : 1)
             float v[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] = p[8 * st + e];
-            split3(v, pp[st]);
+            split3_nearest(v, pp[st]);
         }
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
@@ -1144,7 +1145,7 @@ __global__ void __launch_bounds__(THREADS) prefill_parts_kernel(AttnArgs a, int3
             v[u] = v0[u];
             v[4 + u] = v1[u];
         }
-        split3(v, part);
+        split3_nearest(v, part);
         uint8_t* ko = out + (key >> 5) * parts_block_bytes(HD) + (o >> 1) * 3072 + ((key & 31) + 32 * (o & 1)) * 16;
 #pragma unroll
         for (int h = 0; h < 3; ++h) *reinterpret_cast<bf16x8*>(ko + h * 1024) = part[h];
@@ -1152,7 +1153,7 @@ __global__ void __launch_bounds__(THREADS) prefill_parts_kernel(AttnArgs a, int3
 #pragma unroll
         for (int u = 0; u < 8; ++u)
             v[u] = a.cv[(base + min(k0 + 16 * (oct >> 1) + 4 * (oct & 1) + (u & 3) + 8 * (u >> 2), n_keys - 1)) * HD + d];
-        split3(v, part);
+        split3_nearest(v, part);
         uint8_t* vo = out + (oct >> 2) * parts_block_bytes(HD) + HD / 16 * 3072 +
                       (((oct >> 1) & 1) * (HD / 32) + (d >> 5)) * 3072 + ((d & 31) + 32 * (oct & 1)) * 16;
 #pragma unroll
@@ -1193,7 +1194,7 @@ __global__ void __launch_bounds__(THREADS, HD == 64 ? 2 : 1)
             v[e] = v0[e] * qscale;
             v[4 + e] = v1[e] * qscale;
         }
-        split3(v, qp[s]);
+        split3_nearest(v, qp[s]);
     }
 
     const int32_t n_blocks = min((n_keys + 31) / 32, blocks);
@@ -1261,7 +1262,7 @@ __global__ void __launch_bounds__(THREADS, HD == 64 ? 2 : 1)
             float v[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] = p[8 * st + e];
-            split3(v, pp[st]);
+            split3_nearest(v, pp[st]);
         }
 #pragma unroll
         for (int db = 0; db < DB; ++db) {

@@ -7,6 +7,8 @@
 namespace kt {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -39,6 +41,30 @@ __device__ __forceinline__ void split3(const float (&p)[8], bf16x8 (&part)[3]) {
         const float ra = below_upper(a), rb = below_upper(b);
         m[i] = upper_halves(ra, rb);
         l[i] = upper_halves(below_upper(ra), below_upper(rb));
+    }
+    part[0] = __builtin_bit_cast(bf16x8, h);
+    part[1] = __builtin_bit_cast(bf16x8, m);
+    part[2] = __builtin_bit_cast(bf16x8, l);
+}
+
+// The same with each part the nearest bf16 number to what is left, for products of two split
+// numbers, whose smallest part products are not formed: the rests are unbiased and at most
+// 2^-8 and 2^-17 of the number (cut off, one-signed and up to 2^-7 and 2^-15), so that
+// the three products left out are at most 2^-24 of the product, with an rms of 2^-27 on normal
+// inputs (cut off 2^-21 and 2^-24, always toward zero). As many instructions either way. A
+// number that rounds up to infinity (above 3.39e38) makes a NaN of its lower parts, too.
+__device__ __forceinline__ uint32_t nearest_halves(float lo, float hi) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{lo, hi}), bf16x2));
+}
+__device__ __forceinline__ void split3_nearest(const float (&p)[8], bf16x8 (&part)[3]) {
+    u32x4 h, m, l;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        auto below = [](float v, uint32_t half) { return v - __builtin_bit_cast(float, half); };
+        h[i] = nearest_halves(p[2 * i], p[2 * i + 1]);
+        const float ra = below(p[2 * i], h[i] << 16), rb = below(p[2 * i + 1], h[i] & 0xFFFF0000u);
+        m[i] = nearest_halves(ra, rb);
+        l[i] = nearest_halves(below(ra, m[i] << 16), below(rb, m[i] & 0xFFFF0000u));
     }
     part[0] = __builtin_bit_cast(bf16x8, h);
     part[1] = __builtin_bit_cast(bf16x8, m);

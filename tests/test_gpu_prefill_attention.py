@@ -129,3 +129,26 @@ def test_prefill_attention_infinities(kt, d, tokens):
     assert np.isposinf(third[60:, 3]).all()
     keep = np.setdiff1d(np.arange(60), [20])
     assert normwise_rel(third[keep], want[keep, 2 * d:3 * d]) <= 1e-6
+
+
+@pytest.mark.parametrize("d,tokens", [(64, 70), (128, 70), (64, 200), (128, 200)])
+def test_prefill_attention_of_full_significands(kt, d, tokens):
+    """Scores of one product 64 a * a against 64 a * 1 with a = 1 + 2^-7 - 2^-23, all of whose
+    bits below the first bf16 part are set: cut into parts, not rounded, the products that are
+    left out are 4.7e-7 of the score 65 (in powers of two).
+
+    Bound: a score leaves two fp32 roundings, the largest of its sum at 65, 3.9e-6 each; the
+    weight of the first keys, 2^0.5 / (1 + 2^0.5), moves by its complement times ln 2 of that:
+    2.2e-6 (cut off: 8.7e-6 more)."""
+    a = np.float32(1 + 2.0**-7 - 2.0**-23)
+    scale = np.float32(1.0 / np.sqrt(np.float32(d))) * np.float32(1.4426950408889634)
+    near = np.float32(64 * a / scale) + np.arange(-4, 5, dtype=np.float32) * np.float32(2.0**-15)
+    first = near[near * scale == 64 * a]  # the kernel scales q by this
+    banner("prefill-attention-significands", d, tokens, first.size)
+    q, keys, values = (np.zeros(s, np.float32) for s in ((tokens, d), (1, tokens, d), (1, tokens, d)))
+    q[:, 0] = first[0]
+    keys[0, :, 0] = np.where(np.arange(tokens) % 2 == 0, a, np.float32(1))
+    values[0, ::2] = 1.0
+    err = normwise_rel(_call(kt, q, keys, values, 0, 1), _exact(q, keys, values, 0, 1))
+    print(f"  error {err:.2e}", flush=True)
+    assert err <= 2.2e-6
