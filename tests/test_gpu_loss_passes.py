@@ -51,3 +51,37 @@ def test_scratch_kept_with_the_stream(kt, oracle_lib):
             assert out.item() == want[0]
             assert same_bits(out.hidden_grad.numpy(), want[1]) and same_bits(out.bias_grad.numpy().reshape(-1), want[2])
         stream.destroy()
+
+
+def test_scratch_of_wide_rows(kt):
+    """1024 classes of 8192 inputs: a chunk is 4096 rows, 285 MB of logits, rows and gradients,
+    and a pass one chunk. Two passes take no more than one, and give the halves' gradients:
+    with half the scale of one pass's, the same numbers down to fp32 rounding (the weights of
+    the scale are powers of two)."""
+    from test_gpu_recorded_scratch import _free_bytes
+    rows, k, n = 8192, 8192, 1024
+    banner("fused-ce-wide-rows")
+    rng = np.random.default_rng(8)
+    head = kt.QuantizedLinear(k, n, kt.Quantization(4, 64))
+    head.weight = kt.QuantizedTensor.quantize((rng.standard_normal((k, n), dtype=np.float32) * np.float32(0.02)), k, n, kt.Quantization(4, 64))
+    head.bias = kt.DeviceTensor.zeros((1, n))
+    hidden, targets = rng.standard_normal((rows, k), dtype=np.float32), rng.integers(0, n, rows).astype(np.int32)
+
+    def run(h, t):
+        d = kt.DeviceTensor.from_numpy(h)
+        hg, bg = kt.DeviceTensor.zeros(d.shape), kt.DeviceTensor.zeros((1, n))
+        kt.synchronize()
+        kt.release_scratch()
+        before = _free_bytes()
+        out = kt.fused_cross_entropy_loss(d, head, t, hidden_grad=hg, bias_grad=bg)
+        taken = before - _free_bytes()
+        kt.synchronize()
+        return out.item(), hg.numpy(), bg.numpy(), taken
+
+    loss, hg, bg, taken = run(hidden, targets)
+    halves = [run(hidden[s], targets[s]) for s in (slice(0, 4096), slice(4096, None))]
+    print(f"  {taken >> 20} MB, one chunk {halves[0][3] >> 20} MB", flush=True)
+    assert taken <= 400 << 20
+    assert abs(loss - 0.5 * (halves[0][0] + halves[1][0])) <= 1e-6 * loss
+    assert normwise_rel(hg, 0.5 * np.concatenate([h[1] for h in halves])) <= 1e-6
+    assert normwise_rel(bg, 0.5 * (halves[0][2] + halves[1][2])) <= 1e-6
