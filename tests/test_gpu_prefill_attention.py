@@ -152,3 +152,45 @@ def test_prefill_attention_of_full_significands(kt, d, tokens):
     err = normwise_rel(_call(kt, q, keys, values, 0, 1), _exact(q, keys, values, 0, 1))
     print(f"  error {err:.2e}", flush=True)
     assert err <= 2.2e-6
+
+
+@pytest.mark.parametrize("d,tokens", [(64, 100), (128, 100), (64, 1024), (128, 300)])
+def test_prefill_attention_of_rows_without_numbers(kt, d, tokens):
+    """An infinite value at the third key: every later row of its heads is summed from the fp32
+    values, dealt to all waves, and keeps its other dims' values; rows with a NaN query are
+    left as NaNs. In at most 15 times the ordinary call's time (measured 7; 97 when one wave
+    took a block's rows, lane by lane)."""
+    import time
+    heads, kvh = 8, 2
+    rng = np.random.default_rng(tokens)
+    q = rng.standard_normal((tokens, heads * d)).astype(np.float32)
+    keys, values = (rng.standard_normal((kvh, tokens, d)).astype(np.float32) for _ in range(2))
+    banner("prefill-attention-not-numbers", d, tokens)
+    ref = _exact(q, keys, values, 0, heads)
+
+    def seconds():
+        best = 1e9
+        for _ in range(3):
+            from kotensor_amd import _lib
+            dq, dk, dv, pos, out = *(kt.DeviceBuffer.from_numpy(a) for a in (q, keys, values, np.zeros(1, np.int32))), kt.DeviceBuffer(q.nbytes)
+            kt.synchronize()
+            t = time.perf_counter()
+            for _ in range(5):
+                _lib.call("kt_attention", dq.ptr, tokens, pos.ptr, tokens, dk.ptr, dv.ptr, 0, tokens, heads, kvh, d, out.ptr, None)
+            kt.synchronize()
+            best = min(best, time.perf_counter() - t)
+        return best
+
+    plain = seconds()
+    values[1, 2, 5] = np.inf
+    q[tokens - 1, 5 * d + 7] = np.nan
+    assert seconds() <= 15 * plain
+    got = _call(kt, q, keys, values, 0, heads)
+    assert np.isnan(got[tokens - 1, 5 * d:6 * d]).all()
+    assert normwise_rel(got[:, :4 * d], ref[:, :4 * d]) <= 1e-6  # the other key/value head
+    mine, want = got[:, 4 * d:].reshape(tokens, 4, d).copy(), ref[:, 4 * d:].reshape(tokens, 4, d).copy()
+    mine[tokens - 1, 1], want[tokens - 1, 1] = 0.0, 0.0
+    hit = mine[2:, :, 5]
+    assert np.isposinf(np.delete(hit.reshape(-1), (tokens - 3) * 4 + 1)).all()
+    mine[2:, :, 5], want[2:, :, 5] = 0.0, 0.0
+    assert normwise_rel(mine, want) <= 1e-6

@@ -212,3 +212,70 @@ def test_two_threads_on_one_stream(kt, oracle_lib):
     for t in threads:
         t.join()
     assert all(len(e) == 80 and max(e) <= TOL for e in errors)
+
+
+@pytest.mark.parametrize("bits,m,k,n", [(4, 40, 700, 2001), (8, 70, 1024, 1500), (4, 3, 2300, 4096)])
+def test_transposed_of_rows_without_numbers(kt, oracle_lib, bits, m, k, n):
+    """Many infinite and NaN dY elements: a NaN anywhere in a row makes all of its outputs
+    NaNs; a row with one infinity has its products' signs; a row of infinities of both signs
+    has NaNs where both meet; the other rows keep their bits."""
+    banner("split-transposed-rows", bits, m, k, n)
+    q = _weights(oracle_lib, k, n, bits, 64, m)
+    qt, w = upload_quantized(kt, q), q.dequantize()
+    dy = np.random.default_rng(m).standard_normal((m, n)).astype(np.float32)
+    plain = _transposed(kt, dy, qt)
+    odd = dy.copy()
+    odd[0, ::7] = np.nan
+    odd[1, n - 1] = -np.inf
+    if m > 3:
+        odd[m - 1] = np.inf
+        odd[m // 2:m // 2 + 4, n // 2] = np.nan
+    got = _transposed(kt, odd, qt)
+    assert np.isnan(got[0]).all()
+    with np.errstate(invalid="ignore"):
+        assert np.array_equal(got[1], np.float32(-np.inf) * w[:, n - 1], equal_nan=True)
+        changed = [0, 1]
+        if m > 3:
+            assert np.array_equal(got[m - 1], (np.float32(np.inf) * w).sum(1), equal_nan=True)
+            assert np.isnan(got[m // 2:m // 2 + 4]).all()
+            changed += [m - 1, *range(m // 2, m // 2 + 4)]
+    rest = np.setdiff1d(np.arange(m), changed)
+    assert same_bits(got[rest], plain[rest])
+
+
+def test_rows_without_numbers_take_little_longer(kt, oracle_lib):
+    """A whole input of NaNs or infinities is not summed element by element over all of K or
+    N: at most 8 times the ordinary call's time (measured 2.1 and 5.6 times for the product,
+    2.0 for the transposed one; with every element's whole sum the product took 167)."""
+    import time
+    banner("split-not-numbers-time")
+    m, k, n = 512, 2048, 8191
+
+    def seconds(x, run):
+        a, out = kt.DeviceBuffer.from_numpy(x), kt.DeviceBuffer(4 * m * max(k, n))
+        best = 1e9
+        for _ in range(4):
+            kt.synchronize()
+            t = time.perf_counter()
+            for _ in range(5):
+                run(a, out)
+            kt.synchronize()
+            best = min(best, time.perf_counter() - t)
+        return best
+
+    q = _weights(oracle_lib, k, n, 4, 64, 1)
+    qt = upload_quantized(kt, q)
+    rng = np.random.default_rng(2)
+    forward = lambda a, c: kt.MatMul.multiply_quantized(a, qt, c, m, accumulate=False)  # noqa: E731
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    plain = seconds(x, forward)
+    for v in (np.nan, np.inf):
+        odd = x.copy()
+        odd[:, k // 2] = v
+        assert seconds(odd, forward) <= 8 * plain
+    back = lambda a, c: kt.MatMul.multiply_by_quantized_transposed(a, qt, c, m, accumulate=False)  # noqa: E731
+    dy = rng.standard_normal((m, n)).astype(np.float32)
+    plain = seconds(dy, back)
+    odd = dy.copy()
+    odd[:, n // 2] = np.nan
+    assert seconds(odd, back) <= 8 * plain
