@@ -826,11 +826,16 @@ int32_t launch_transposed_split(const float* dy, int32_t m, const WeightView& w,
     return status;
 }
 
-// generic_matmul (kt_misc.hip: one thread per output, k in sequence) stays where the product
-// is a few rows of one step (M = 3, 64 -> 70: 10.0 us with the call against 12.8 here; M = 2,
-// 128 -> 100 18.8 against 12.6).
+// generic_matmul (kt_misc.hip: one thread per output, k in sequence: 0.13 to 0.16 us a k up to
+// about 4000 waves, more with their number) stays for short sums, where this kernel's 12 to
+// 17 us of a step or two are longer. Generic / here, with the call, INT4: 64 rows 32 -> 70
+// 5.8 / 15.0 us, 64 -> 70 9.6 / 13.9, 80 -> 257 14.5 / 15.3, 88 -> 70 12.6 / 14.6, 96 -> 257
+// 16.9 / 15.3; 1000 rows 64 -> 257 14.5 / 13.5, 64 -> 999 26 / 14; 4000 rows 48 -> 70 15.0 /
+// 15.8, 64 -> 70 19 / 14; 16 rows 80 -> 257 14.3 / 14.5, 88 -> 257 15.6 / 14.5; one row
+// 64 -> 70 9.1 / 12, 72 -> 257 12.2 / 12.4, 80 -> 257 13.4 / 12.5.
 bool forward_split_preferred(int32_t m, const WeightView& w) {
-    if (w.K <= STEP && m <= 16) return false;
+    const int64_t waves = static_cast<int64_t>(m) * ceil_div(w.N, 64);  // of generic_matmul
+    if (w.K <= (m > 16 ? 88 : m > 4 ? 80 : 72) && w.K * waves <= 410 << 10) return false;
     // 32 k share a scale, the clamped loads lie in a row; 32-bit lane offsets
     return w.g % 32 == 0 && w.N >= 8 && w.K <= 1 << 22 && w.bpr <= 1 << 24;
 }

@@ -279,3 +279,43 @@ def test_rows_without_numbers_take_little_longer(kt, oracle_lib):
     odd = dy.copy()
     odd[:, n // 2] = np.nan
     assert seconds(odd, back) <= 8 * plain
+
+
+# both sides of where generic_matmul's short sums end: K at each number of rows, K times its waves
+@pytest.mark.parametrize("m,k,n,bits,g,generic", [
+    (17, 88, 257, 4, 64, True), (17, 89, 257, 4, 64, False), (16, 80, 70, 8, 32, True), (16, 81, 70, 8, 32, False),
+    (4, 72, 999, 4, 64, True), (4, 73, 999, 4, 64, False), (410, 64, 1001, 4, 32, True), (411, 64, 1001, 4, 32, False),
+    (33, 97, 65, 8, 32, False), (65, 95, 515, 8, 64, False),
+])
+def test_forward_where_short_sums_end(kt, oracle_lib, m, k, n, bits, g, generic):
+    """generic_matmul adds up to 88 products a row's group, sum a q - zero sum a: a walk of
+    nine roundings of 2^-24, which the difference enlarges up to four times: 2.2e-6."""
+    banner("split-forward-short", m, k, n, bits, g)
+    q = _weights(oracle_lib, k, n, bits, g, m + k + n)
+    x = np.random.default_rng(m).standard_normal((m, k)).astype(np.float32)
+    a, c = kt.DeviceBuffer.from_numpy(x), kt.DeviceBuffer(m * n * 4)
+    kt.MatMul.multiply_quantized(a, upload_quantized(kt, q), c, m, accumulate=False)
+    kt.synchronize()
+    got, want = c.download(np.float32).reshape(m, n), x.astype(np.float64) @ q.dequantize().astype(np.float64)
+    err = (np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)).max()
+    print(f"  largest row error {err:.2e}", flush=True)
+    assert err <= (2.2e-6 if generic else TOL)
+
+
+def test_short_sums_of_more_rows(kt, oracle_lib):
+    """64 -> 70: 17 rows take what 16 do (one launch of generic_matmul, 9.5 us; 13.4 in this
+    file's kernel), with a quarter for the clock."""
+    import time
+    banner("split-short-sums-time")
+    q = upload_quantized(kt, _weights(oracle_lib, 64, 70, 4, 64, 3))
+    a, c = kt.DeviceBuffer.from_numpy(np.ones((17, 64), np.float32)), kt.DeviceBuffer(17 * 70 * 4)
+    best = {16: 1e9, 17: 1e9}
+    for _ in range(8):
+        for m in best:
+            kt.synchronize()
+            t = time.perf_counter()
+            for _ in range(200):
+                kt.MatMul.multiply_quantized(a, q, c, m, accumulate=False)
+            kt.synchronize()
+            best[m] = min(best[m], time.perf_counter() - t)
+    assert best[17] <= 1.25 * best[16]
