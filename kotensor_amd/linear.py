@@ -9,7 +9,7 @@ import numpy as np
 
 from . import _lib
 from .device import DeviceBuffer, Stream, default_stream
-from .matmul import DeviceTensor, _call_group
+from .matmul import DeviceTensor, _call_group, _ptr
 from .quantization import Quantization, QuantizedTensor
 
 
@@ -73,16 +73,24 @@ def forward_into_group(layers, x: DeviceTensor, outs, stream: Stream | None = No
     """``outs[i] = x · deq(layers[i].weight) + layers[i].bias`` for projections of one input
     (wQ/wK/wV, Attention.kt:220-222; wGate/wUp, SwiGLU.kt:19-25), one launch per four layers."""
     m, k = x.shape
+    structs, outputs, biases = [], [], []
     for layer, out in zip(layers, outs):
+        n, buffer, bias = layer.out_size, out.buffer, layer.bias
         if layer.in_size != k:
             raise _lib.IllegalArgumentException(f"{k} != {layer.in_size}")
-        if out.shape != (m, layer.out_size):
-            raise _lib.IllegalArgumentException(f"out shape {list(out.shape)} != [{m}, {layer.out_size}]")
+        if out.shape != (m, n):
+            raise _lib.IllegalArgumentException(f"out shape {list(out.shape)} != [{m}, {n}]")
+        if buffer.nbytes < m * n * 4:
+            raise _lib.IllegalArgumentException(f"output has {buffer.nbytes // 4} elements, needs {m} × {n}")
+        structs.append(layer.weight.qweight)
+        outputs.append(buffer._ptr)
+        biases.append(bias.buffer._ptr if type(bias) is DeviceTensor else _ptr(bias))
     if len(layers) != len(outs):
         raise _lib.IllegalArgumentException("weights, outputs and biases differ in length")
-    if layers:  # (a tensor's buffer holds its shape: nothing more to check)
-        _call_group(x.buffer._ptr, m, [l._weight._struct for l in layers], [o.buffer._ptr for o in outs],
-                    [None if l.bias is None else l.bias.buffer._ptr for l in layers], 0, 1.0, stream)
+    if structs:
+        if x.buffer.nbytes < m * k * 4:
+            raise _lib.IllegalArgumentException(f"a has {x.buffer.nbytes // 4} elements, needs {m} × {k}")
+        _call_group(x.buffer._ptr, m, structs, outputs, biases, 0, 1.0, stream)
     return outs
 
 
