@@ -1612,7 +1612,8 @@ static int32_t attention_launch(const float* q, int32_t tokens, const int32_t* p
         return fail(KT_ERR_ARGUMENT, "attention: q and the caches must be 16-byte aligned");
     if (tokens == 0) return KT_OK;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (!k_new && tokens >= PREFILL_MIN_TOKENS && (head_dim == 64 || head_dim == 128) && G <= PQ_ROWS) {
+    if (!k_new && tokens >= PREFILL_MIN_TOKENS && (head_dim == 64 || head_dim == 128)) {
+        static_assert(MAX_NACC * THREADS / 64 <= SPLIT_ROWS && SPLIT_ROWS <= PQ_ROWS, "a block holds a token's heads");
         // many tokens: the query-blocked MFMA kernel
         AttnArgs a{};
         a.q = q;
@@ -1629,7 +1630,7 @@ static int32_t attention_launch(const float* q, int32_t tokens, const int32_t* p
         a.splits = 1;
         const size_t parts_bytes = static_cast<size_t>(num_kv_heads) * 2 * ceil_div(key_bound, PKT) *
                                    (head_dim == 64 ? parts_block_bytes(64) : parts_block_bytes(128));
-        if (key_bound >= PARTS_MIN_KEYS && parts_bytes <= PARTS_LIMIT && G <= SPLIT_ROWS) {
+        if (key_bound >= PARTS_MIN_KEYS && parts_bytes <= PARTS_LIMIT) {
             CallScratch parts;
             if (const int32_t status = parts.take(st, parts_bytes)) return status;
             if (parts.ptr)
