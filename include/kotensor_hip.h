@@ -258,11 +258,11 @@ int32_t kt_qmatmul_transposed(const float* dy, int32_t m, const kt_qweight* w, f
  * - l[target], l = hidden . deq(W) + bias. hidden_grad [rows x K] and bias_grad [N]
  * (device, each may be NULL) receive d loss / d hidden and d loss / d bias, added to
  * what they hold when accumulate != 0 (ignored rows get 0). Rows go through in chunks of
- * 2^22 / N rows as in the reference, as many chunks at a time as 2^25 floats (128 MB)
- * hold with N + 2 K a row (one, if the memory for more is not left: the sums are then of
- * another order); scratch for them is allocated and freed on the stream, from a pool that
- * keeps up to 256 MB (see kt_stream_destroy). Asynchronous. KT_ERR_ARGUMENT for no rows or a
- * target out of range ("target t out of bounds N"). */
+ * 2^22 / N rows as in the reference, as many chunks at a time as 2^25 logits (128 MB)
+ * and 2^25 floats of rows and their gradients (2 K a row) hold (one, if the memory for more
+ * is not left: the sums are then of another order); scratch for them is allocated and freed
+ * on the stream, from a pool that keeps up to 256 MB (see kt_stream_destroy). Asynchronous.
+ * KT_ERR_ARGUMENT for no rows or a target out of range ("target t out of bounds N"). */
 int32_t kt_fused_cross_entropy(const float* hidden, int32_t rows, const kt_qweight* head, const float* bias,
                                const int32_t* targets, int32_t ignore_index, float* loss, float* hidden_grad,
                                float* bias_grad, int32_t accumulate, void* stream);

@@ -8,8 +8,8 @@
 // Loss.kt:129-133, :236-260): a chunk's rows, and with them the kernel that makes its
 // logits, do not depend on how many ignored rows lie between them. The reference takes a
 // chunk at a time to bound the logits' memory; here a pass holds as many whole chunks as
-// 2^25 floats (128 MB) of logits, gathered rows and their gradients, so that every kernel
-// fills the GPU; one chunk where that much memory is not left. Per pass: the logits by
+// 2^25 logits (128 MB), and 2^25 floats of gathered rows and their gradients, so that every
+// kernel fills the GPU; one chunk where that much memory is not left. Per pass: the logits by
 // kt_qmatmul (the prefill GEMM or the small-M kernels, with the bias), one workgroup per
 // row for the row's max, sum of exponentials, loss and (in place) its logit gradients
 // scale * (softmax - onehot) (logitGradients, Loss.kt:275-291), then the bias gradient as
@@ -214,7 +214,8 @@ extern "C" int32_t kt_fused_cross_entropy(const float* hidden, int32_t rows, con
     }
     const int32_t chunk = std::max(1, std::min(FUSED_CHUNK_ELEMENTS / V, active));  // chunkRows
     const int64_t row_floats = V + 2 * static_cast<int64_t>(K);
-    int32_t pass = std::min<int64_t>(std::max<int64_t>(1, PASS_ELEMENTS / row_floats / chunk) * chunk, active);
+    const int64_t fit = PASS_ELEMENTS / std::max<int64_t>(V, 2 * static_cast<int64_t>(K));  // rows
+    int32_t pass = std::min<int64_t>(std::max<int64_t>(1, fit / chunk) * chunk, active);
     // device scratch of this call: the pass's logits, its gathered rows and their hidden
     // gradient, the per-row losses, the active rows' indices and targets
     const size_t list_bytes = static_cast<size_t>(active) * (sizeof(float) + 2 * sizeof(int32_t));
