@@ -116,9 +116,9 @@ int32_t kt_memset(void* dst, int32_t value, size_t bytes, void* stream);
 int32_t kt_stream_create(void** stream);
 /* Besides the stream itself gives back the scratch memory that calls on it kept. For NULL
  * it waits for the device and gives back what the library keeps between calls as scratch
- * of the split products and the prompt attention, for the null stream and any other (also
- * streams that their owner destroyed): up to 64 MB a stream, and up to 256 MB a device in
- * a pool that the fused loss's scratch comes from too. Later calls take it anew. */
+ * of the split products, the prompt attention (up to 64 MB a stream) and the fused loss
+ * (up to 192 MB a stream), for the null stream and any other, also streams that their
+ * owner destroyed. Later calls take it anew. */
 int32_t kt_stream_destroy(void* stream);
 /* kt_stream_sync and kt_memcpy_d2h (which synchronizes) also report a bounded wait
  * inside a kernel that gave up since the stream's last synchronization (the chained
@@ -260,9 +260,10 @@ int32_t kt_qmatmul_transposed(const float* dy, int32_t m, const kt_qweight* w, f
  * what they hold when accumulate != 0 (ignored rows get 0). Rows go through in chunks of
  * 2^22 / N rows as in the reference, as many chunks at a time as 2^25 logits (128 MB)
  * and 2^25 floats of rows and their gradients (2 K a row) hold (one, if the memory for more
- * is not left: the sums are then of another order); scratch for them is allocated and freed
- * on the stream, from a pool that keeps up to 256 MB (see kt_stream_destroy). Asynchronous.
- * KT_ERR_ARGUMENT for no rows or a target out of range ("target t out of bounds N"). */
+ * is not left: the sums are then of another order); scratch of up to 192 MB stays for the
+ * stream's next call (see kt_stream_destroy), larger scratch, and any under capture, is
+ * allocated and freed on the stream. Asynchronous. KT_ERR_ARGUMENT for no rows or a
+ * target out of range ("target t out of bounds N"). */
 int32_t kt_fused_cross_entropy(const float* hidden, int32_t rows, const kt_qweight* head, const float* bias,
                                const int32_t* targets, int32_t ignore_index, float* loss, float* hidden_grad,
                                float* bias_grad, int32_t accumulate, void* stream);

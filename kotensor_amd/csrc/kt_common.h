@@ -72,8 +72,10 @@ bool workspace_present(hipStream_t stream);
 // at most POOL_KEPT bytes stay in the pool when nothing uses them (scratch_release and
 // kt_stream_destroy give them back).
 //
-// take: an area that stays for the next call (the split products' slices, the prefill
-// attention's parts; getting memory from the pool for each call costs 10 us of host time).
+// take: an area that stays for the next call: CALL_SLICES for the split products' slices and
+// the prefill attention's parts, CALL_LOSS for the fused loss, whose products want the other.
+// (Getting memory from the pool for each call costs 10 us of host time, and 300 us where a
+// hipFree in between has emptied the pool.)
 // Another thread's call that wants the same area waits until this one has enqueued its
 // launches, so they never interleave on it. An eager call takes the area of its stream; a
 // call recorded between kt_graph_begin and kt_graph_end takes one that belongs to the graph
@@ -84,8 +86,10 @@ bool workspace_present(hipStream_t stream);
 // what a call takes depends on its shapes alone. (Calls on a caller's fixed workspace get its
 // general area, which holds SLICES_LIMIT bytes.)
 //
-// allocate: memory for this call only, freed on the stream behind its launches (the fused
-// loss); ptr stays null if there is none left. In a capture it becomes part of the graph.
+// allocate: memory for this call only, freed on the stream behind its launches (a loss's of
+// more than LOSS_LIMIT); ptr stays null if there is none left. In a capture it becomes part of
+// the graph.
+enum CallArea { CALL_SLICES, CALL_LOSS, CALL_AREAS };
 struct Area {
     void* ptr = nullptr;
     size_t bytes = 0;
@@ -97,7 +101,7 @@ class CallScratch {
     CallScratch(const CallScratch&) = delete;
     CallScratch& operator=(const CallScratch&) = delete;
     ~CallScratch();  // after the call's last launch is enqueued
-    int32_t take(hipStream_t stream, size_t bytes);
+    int32_t take(CallArea kind, hipStream_t stream, size_t bytes);
     int32_t allocate(hipStream_t stream, size_t bytes);
     void* ptr = nullptr;
 
@@ -117,6 +121,7 @@ constexpr size_t SCRATCH_BYTES = size_t(64) << 20;
 constexpr size_t SCRATCH_ZERO_BYTES = size_t(4) << 20;
 constexpr size_t SLICES_LIMIT = SCRATCH_BYTES - SCRATCH_ZERO_BYTES - COUNTER_BYTES;
 constexpr size_t PARTS_LIMIT = size_t(64) << 20;
+constexpr size_t LOSS_LIMIT = size_t(192) << 20;
 
 // Validated view of a kt_qweight, with the derived layout numbers.
 struct WeightView {

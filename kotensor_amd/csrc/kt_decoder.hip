@@ -1632,7 +1632,7 @@ static int32_t attention_launch(const float* q, int32_t tokens, const int32_t* p
                                    (head_dim == 64 ? parts_block_bytes(64) : parts_block_bytes(128));
         if (key_bound >= PARTS_MIN_KEYS && parts_bytes <= PARTS_LIMIT) {
             CallScratch parts;
-            if (const int32_t status = parts.take(st, parts_bytes)) return status;
+            if (const int32_t status = parts.take(CALL_SLICES, st, parts_bytes)) return status;
             if (parts.ptr)
                 return head_dim == 64 ? launch_prefill_parts<64>(a, tokens, key_bound, static_cast<uint8_t*>(parts.ptr), st)
                                       : launch_prefill_parts<128>(a, tokens, key_bound, static_cast<uint8_t*>(parts.ptr), st);

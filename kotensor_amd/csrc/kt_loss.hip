@@ -219,11 +219,17 @@ extern "C" int32_t kt_fused_cross_entropy(const float* hidden, int32_t rows, con
     // device scratch of this call: the pass's logits, its gathered rows and their hidden
     // gradient, the per-row losses, the active rows' indices and targets
     const size_t list_bytes = static_cast<size_t>(active) * (sizeof(float) + 2 * sizeof(int32_t));
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    KT_HIP(hipStreamIsCapturing(st, &capture));
     CallScratch area;
-    if ((status = area.allocate(st, pass * row_floats * sizeof(float) + list_bytes))) return status;
+    auto get = [&]() {
+        const size_t bytes = pass * row_floats * sizeof(float) + list_bytes;
+        return capture == hipStreamCaptureStatusNone && bytes <= LOSS_LIMIT ? area.take(CALL_LOSS, st, bytes) : area.allocate(st, bytes);
+    };
+    if ((status = get())) return status;
     if (!area.ptr && pass > chunk) {
         pass = chunk;
-        if ((status = area.allocate(st, pass * row_floats * sizeof(float) + list_bytes))) return status;
+        if ((status = get())) return status;
     }
     if (!area.ptr) return hip_fail(hipErrorOutOfMemory, "fused cross-entropy: scratch");
     const size_t logit_bytes = static_cast<size_t>(pass) * V * sizeof(float);

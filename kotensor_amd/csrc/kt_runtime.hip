@@ -43,12 +43,12 @@ struct Block {
 std::mutex g_ws_mutex;
 std::map<std::pair<int, hipStream_t>, Block> g_ws;
 // The areas of the streams' eager calls (CallScratch), from g_pools.
-std::map<std::pair<int, hipStream_t>, std::shared_ptr<Area>> g_areas;
+std::map<std::pair<int, hipStream_t>, std::shared_ptr<Area>> g_areas[CALL_AREAS];
 // The areas of recorded calls, while their capture runs (by its id) and once it is a graph:
 // the graph's end frees them.
 struct Capture {
     hipStream_t origin = nullptr;  // the stream of kt_graph_begin
-    std::map<hipStream_t, std::shared_ptr<Area>> areas;
+    std::map<hipStream_t, std::shared_ptr<Area>> areas[CALL_AREAS];
     std::vector<void*> blocks;     // all that the recorded calls may address
 };
 std::map<unsigned long long, Capture> g_captures;
@@ -211,7 +211,7 @@ void pool_trim() {
 }
 }  // namespace
 
-int32_t CallScratch::take(hipStream_t stream, size_t bytes) {
+int32_t CallScratch::take(CallArea kind, hipStream_t stream, size_t bytes) {
     if (t_fixed) {
         const size_t head = COUNTER_BYTES + t_fixed->zero_bytes;
         if (bytes <= t_fixed->bytes - head) ptr = t_fixed->ptr + head;
@@ -232,14 +232,14 @@ int32_t CallScratch::take(hipStream_t stream, size_t bytes) {
             if (it == g_captures.end()) return KT_OK;
             capture = &it->second;
         }
-        std::shared_ptr<Area>& slot = capture ? capture->areas[stream] : g_areas[std::make_pair(device, stream)];
+        std::shared_ptr<Area>& slot = capture ? capture->areas[kind][stream] : g_areas[kind][std::make_pair(device, stream)];
         if (!slot) slot = std::make_shared<Area>();
         area = slot;
         if (!area->busy) break;
         g_area_free.wait(lock);  // another thread is enqueuing with it
     }
     if (area->bytes < bytes) {
-        const size_t want = std::min(bytes + bytes / 4, std::max(bytes, PARTS_LIMIT));
+        const size_t want = std::min(bytes + bytes / 4, std::max(bytes, kind == CALL_LOSS ? LOSS_LIMIT : PARTS_LIMIT));
         if (capture) {  // a smaller block stays with the graph, whose earlier calls use it
             *area = Area{};
             RelaxedCapture relaxed;
@@ -296,14 +296,15 @@ int32_t scratch_release() {
     {
         std::lock_guard<std::mutex> lock(g_ws_mutex);
         KT_HIP(hipDeviceSynchronize());
-        for (auto it = g_areas.begin(); it != g_areas.end();) {
-            if (it->first.first != device || it->second->busy) {
-                ++it;
-                continue;
+        for (auto& areas : g_areas)
+            for (auto it = areas.begin(); it != areas.end();) {
+                if (it->first.first != device || it->second->busy) {
+                    ++it;
+                    continue;
+                }
+                if (it->second->ptr) KT_HIP(hipFreeAsync(it->second->ptr, nullptr));
+                it = areas.erase(it);
             }
-            if (it->second->ptr) KT_HIP(hipFreeAsync(it->second->ptr, nullptr));
-            it = g_areas.erase(it);
-        }
     }
     KT_HIP(hipStreamSynchronize(nullptr));
     pool_trim();
@@ -638,10 +639,11 @@ int32_t kt_stream_destroy(void* stream) {
             else if (it->second.ptr) KT_HIP(hipFree(it->second.ptr));
             g_ws.erase(it);
         }
-        const auto area = g_areas.find(std::make_pair(device, s));
-        if (area != g_areas.end()) {
+        for (auto& areas : g_areas) {
+            const auto area = areas.find(std::make_pair(device, s));
+            if (area == areas.end()) continue;
             if (area->second->ptr) KT_HIP(hipFreeAsync(area->second->ptr, s));
-            g_areas.erase(area);
+            areas.erase(area);
         }
     }
     KT_HIP(hipStreamSynchronize(s));

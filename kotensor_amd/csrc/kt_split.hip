@@ -794,7 +794,7 @@ int32_t launch_transposed_split(const float* dy, int32_t m, const WeightView& w,
     choose_slices(tiles, p.steps, slice, &p.splits, &p.steps_per_split);
     CallScratch area;
     if (p.splits > 1) {
-        if (const int32_t status = area.take(st, p.splits * slice)) return status;
+        if (const int32_t status = area.take(CALL_SLICES, st, p.splits * slice)) return status;
         if (area.ptr) {
             p.out = static_cast<float*>(area.ptr);
         } else {
@@ -853,7 +853,7 @@ int32_t launch_forward_split(const float* a, int32_t m, const WeightView& w, flo
     choose_slices(tiles, p.steps, slice, &p.splits, &p.steps_per_split);
     CallScratch area;
     if (p.splits > 1) {
-        if (const int32_t status = area.take(st, p.splits * slice)) return status;
+        if (const int32_t status = area.take(CALL_SLICES, st, p.splits * slice)) return status;
         if (area.ptr) {
             p.c = static_cast<float*>(area.ptr);
         } else {  // no scratch to have (CallScratch): one slice (3 us a step of 64 k; generic_matmul 9)

@@ -85,3 +85,26 @@ def test_scratch_of_wide_rows(kt):
     assert abs(loss - 0.5 * (halves[0][0] + halves[1][0])) <= 1e-6 * loss
     assert normwise_rel(hg, 0.5 * np.concatenate([h[1] for h in halves])) <= 1e-6
     assert normwise_rel(bg, 0.5 * (halves[0][2] + halves[1][2])) <= 1e-6
+
+
+def test_two_threads_on_one_stream(kt, oracle_lib):
+    """Two threads' losses on the null stream, in one area one after the other: always the bits
+    each has alone."""
+    import threading
+    banner("fused-ce-two-threads")
+    cases = [_setup(kt, oracle_lib, 64, n, rows, 4, 64, n) for n, rows in ((2000, 40), (3001, 130))]
+    want = [_run(kt, head, hidden, targets) for _, head, _, hidden, targets in cases]
+    bad = []
+
+    def work(i):
+        _, head, _, hidden, targets = cases[i]
+        for _ in range(20):
+            got = _run(kt, head, hidden, targets)
+            bad.append(got[0] != want[i][0] or not same_bits(got[1], want[i][1]) or not same_bits(got[2], want[i][2]))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(bad) == 40 and not any(bad)
