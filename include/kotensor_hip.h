@@ -9,10 +9,11 @@
  *     by the caller (kt_dev_alloc / kt_dev_free). The library never frees them.
  *   - Entry points are stateless and reentrant. Compute entry points enqueue work on
  *     the given stream and return before it finishes, except kt_quantize (see there).
- *     The library keeps one internal workspace per (device, stream); calls that
- *     share a stream are ordered by it, and calls on different streams never share
- *     one, with one exception: every kt_qmatmul_noalloc call on a device uses that
- *     device's single fixed array (see there), so such calls must not overlap.
+ *     The library keeps one internal workspace per (device, stream), and scratch areas
+ *     beside it (see kt_graph_begin); calls that share a stream are ordered by it, and
+ *     calls on different streams never share one, with one exception: every
+ *     kt_qmatmul_noalloc call on a device uses that device's single fixed array (see
+ *     there), so such calls must not overlap.
  *   - Return value: KT_OK (0) on success; a negative KT_ERR_* for an argument error
  *     (the reference raises IllegalArgumentException for the same cases) except
  *     KT_ERR_STATE; a positive value is a HIP runtime error code (the reference has no
@@ -246,7 +247,8 @@ int32_t kt_qmatmul_group(const float* a, int32_t m, const kt_qweight* weights, i
 /* MatMul.multiplyByQuantizedTransposed(dy, weight, dx, m, accumulate),
  * K/MatMul.kt:954-981:  dx[m x K] = (accumulate ? dx : 0) + dy[m x N] . deq(W)^T.
  * 8-bit rows are dequantized without zero points, as dequantizeRow does
- * (K/QuantizedTensor.kt:198-202). Asynchronous. */
+ * (K/QuantizedTensor.kt:198-202). May hold scratch for slices of the sum (see
+ * kt_graph_begin). Asynchronous. */
 int32_t kt_qmatmul_transposed(const float* dy, int32_t m, const kt_qweight* w, float* dx,
                               int32_t accumulate, void* stream);
 
@@ -315,7 +317,9 @@ int32_t kt_rope_kv(float* q, float* k, const float* v, int32_t tokens, int32_t n
  * For fewer than 16 tokens the keys are split over workgroups whose partials meet in the
  * stream's workspace (its zeroed region, zero again when the launch ends); as for every
  * call that takes the workspace, a graph is recorded after one eager call of the same
- * shapes on the stream. */
+ * shapes on the stream. One token of head dimension 64 with a key bound of at most 640 has
+ * no splits and needs none. 16 and more tokens over 192 and more keys may hold scratch for
+ * the keys and values (see kt_graph_begin). */
 int32_t kt_attention(const float* q, int32_t tokens, const int32_t* position, int32_t key_bound,
                      const float* cache_k, const float* cache_v, int32_t layer, int32_t max_seq,
                      int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, float* context,

@@ -838,9 +838,9 @@ __global__ void __launch_bounds__(64 * DIRECT_WAVES) attention_direct_kernel(Att
 //     the rescaled running sum with one multiply-add.
 // The longest blocks go out first, the shortest with them while two workgroups per CU hold
 // all (workgroups y and y + 32 of an XCD share a CU: the pair is then about as long as any).
-// 1024 tokens, 32 query and 8 kv heads of 64: 44 us (fp32 matrix instructions on 128 rows a
-// workgroup: 103 us), head dimension 128 119 us (184), 64 tokens after 1024 44 us (107);
-// error against 64 bits 1.4e-7 (3.3e-7). Bound by the longest block's chain of tiles: about
+// 1024 tokens, 32 query and 8 kv heads of 64: 50 us traced (fp32 matrix instructions on 128 rows a
+// workgroup: 109), with the call head dimension 128 119 us (184), 64 tokens after 1024 44 (107);
+// error against 64 bits 1.2e-7 (3.3e-7). Bound by the longest block's chain of tiles: about
 // 565 vector instructions and 48 matrix products a wave and tile, which overlap only where
 // two workgroups share the CU.
 constexpr int PQ_ROWS = 64;   // query rows per workgroup
@@ -1175,7 +1175,7 @@ __global__ void __launch_bounds__(THREADS, HD == 64 ? 2 : 1)
 // Per query row the tile kernel above also splits every key and value; here a wave and block
 // has about 345 vector instructions beside its 48 matrix products, and 24 KiB of operands
 // from L2. Traced (tile kernel -> this with its 5 us of splitting): 1024 tokens, 32 query and
-// 8 kv heads of 64 48 -> 42 us; with the call 512 tokens 25 -> 19, 64 after 1024 44 -> 21, 17
+// 8 kv heads of 64 50 -> 43 us; with the call 512 tokens 25 -> 19, 64 after 1024 44 -> 21, 17
 // after 900 40 -> 19; heads of 128 1024 tokens 118 -> 84. Short contexts stay with the tile
 // kernel's one launch (100 tokens, 14 heads: 9.6 against 15 us; 200 of 128 dims 26 against 18),
 // so do calls whose parts exceed PARTS_LIMIT, and those that get no area (CallScratch).

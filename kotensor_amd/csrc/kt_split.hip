@@ -101,8 +101,9 @@ struct SplitArgs {
 // the row-by-row kernel 1.26e-7).
 // Bound by vector ALU work: about 700 instructions per wave and step, two thirds of them the
 // splits, beside 48 matrix products (35% of the matrix units' time). M = 512, K = 2048,
-// N = 8192, INT4 g = 64: 76 us, 220 TFLOP/s, plus 8 us for the slices' sum (row by row on
-// the vector ALU: 2850 us); g = 128 63 us, g = 32 96 us.
+// N = 8192, INT4: the call with the slices' sum 76 us at g = 64, 226 TFLOP/s (row by row on
+// the vector ALU: 2850 us), 70 at g = 128, 97 at g = 32; traced one by one the two kernels
+// take 75.7 and 8.6 us.
 template <int BITS, int WM, int GB>
 __global__ void __launch_bounds__(THREADS, 2) transposed_split_kernel(SplitArgs p) {
     constexpr int WK = 4 / WM, TK = 128 * WK, GW = 4 / GB, GT = WK * GW;
@@ -458,8 +459,8 @@ struct ForwardArgs {
 // scaled, with one fp32 multiply-add: SC steps of 16 k share a scale (4 or 2).
 // Bound by the steps' conversions and splits (vector ALU, 350 instructions a wave and step)
 // beside 48 matrix products, at few rows by the conversions and the slices' sum:
-// M = 512, 2048 -> 8191, INT4 g = 64 80 us, 214 TFLOP/s (generic_matmul 2784 us); M = 37,
-// 1000 -> 2999 19 us with the call (163); M = 1, 14336 -> 20001 INT8 132 us, 2.2 TB/s (5104).
+// M = 512, 2048 -> 8191, INT4 g = 64 75 to 81 us, 220 TFLOP/s (generic_matmul 2784 us); M = 37,
+// 1000 -> 2999 18 us with the call (163); M = 1, 14336 -> 20001 INT8 120 us, 2.4 TB/s (5104).
 template <int BITS, bool ZP, int WM, int SC>
 __global__ void __launch_bounds__(THREADS, 2) forward_split_kernel(ForwardArgs p) {
     constexpr int WN = 4 / WM, TN = 128 * WN;

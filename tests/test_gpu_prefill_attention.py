@@ -3,8 +3,8 @@ against 64 bits. Prefill: blocks of query rows that end inside a token's heads, 
 with every kind of end, a wave without keys of its own, both orders of the blocks, both head
 dimensions; and rows with infinities.
 
-Bound: six products of parts per element leave an fp32 rounding each; with the fp32 sums of
-up to 1600 keys and the exponential's rounding the result is held to 1e-6 normwise."""
+Bound: the six products of parts per element leave out at most an fp32 rounding (2^-24 of the
+product, as often above as below); with the fp32 sums of up to 1600 keys and the exponential's rounding the result is held to 1e-6 normwise."""
 import numpy as np
 import pytest
 
@@ -56,9 +56,8 @@ def test_prefill_attention_against_64_bits(kt, tokens, start, heads, kvh, d):
 
 
 def test_prefill_attention_recorded_without_workspace(kt):
-    """Recorded on a stream that never ran eagerly there is no workspace for the parts: the
-    kernel that splits tiles itself runs; its replays equal the 64-bit result, with eager
-    calls (on parts) in between."""
+    """Recorded on a stream that never ran eagerly (the graph has an area of its own for the
+    parts): replays equal the 64-bit result, with eager calls in between."""
     import ctypes
 
     from kotensor_amd import _lib

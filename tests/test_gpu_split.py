@@ -148,7 +148,7 @@ def test_transposed_infinities_and_nans(kt, oracle_lib):
 
 
 def test_transposed_recorded_without_workspace(kt, oracle_lib):
-    """Recorded on a stream that never ran eagerly (no workspace to split into): replays
+    """Recorded on a stream that never ran eagerly (the graph has scratch of its own): replays
     equal the 64-bit result, with eager calls in between."""
     from kotensor_amd import _lib
     m, k, n = 64, 1024, 2000
@@ -181,7 +181,7 @@ def test_transposed_recorded_without_workspace(kt, oracle_lib):
 
 def test_two_threads_on_one_stream(kt, oracle_lib):
     """Two threads call the sliced products on the null stream at once: the slices' area
-    belongs to one enqueuing call at a time (the other runs one slice)."""
+    belongs to one enqueuing call at a time (the other waits for its launches)."""
     import threading
 
     operands = []
