@@ -211,6 +211,20 @@ void pool_trim() {
 }
 }  // namespace
 
+// Takes the blocks of the calls recorded since kt_graph_begin on `origin`. With g_ws_mutex held.
+static std::vector<void*> captured_blocks(hipStream_t origin) {
+    std::vector<void*> blocks;
+    for (auto it = g_captures.begin(); it != g_captures.end();) {
+        if (it->second.origin != origin) {
+            ++it;
+            continue;
+        }
+        blocks.insert(blocks.end(), it->second.blocks.begin(), it->second.blocks.end());
+        it = g_captures.erase(it);
+    }
+    return blocks;
+}
+
 int32_t CallScratch::take(CallArea kind, hipStream_t stream, size_t bytes) {
     if (t_fixed) {
         const size_t head = COUNTER_BYTES + t_fixed->zero_bytes;
@@ -291,6 +305,7 @@ CallScratch::~CallScratch() {
 }
 
 int32_t scratch_release() {
+    RelaxedCapture relaxed;
     int device = 0;
     KT_HIP(hipGetDevice(&device));
     {
@@ -671,6 +686,7 @@ int32_t kt_graph_begin(void* stream) {
     unsigned long long id = 0;
     if (hipStreamGetCaptureInfo(st, &status, &id) == hipSuccess && status == hipStreamCaptureStatusActive) {
         std::lock_guard<std::mutex> lock(g_ws_mutex);
+        for (void* b : captured_blocks(st)) g_retired.push_back(b);  // of a capture that the caller ended
         g_captures[id].origin = st;
     }
     return KT_OK;
@@ -680,17 +696,12 @@ int32_t kt_graph_end(void* stream, void** graph) {
     if (!stream || !graph) return fail(KT_ERR_ARGUMENT, "stream or graph is NULL");
     *graph = nullptr;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    std::vector<void*> blocks;  // of the calls recorded since kt_graph_begin
-    {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    KT_HIP(hipStreamIsCapturing(st, &status));
+    std::vector<void*> blocks;
+    if (status != hipStreamCaptureStatusNone) {
         std::lock_guard<std::mutex> lock(g_ws_mutex);
-        for (auto it = g_captures.begin(); it != g_captures.end();) {
-            if (it->second.origin != st) {
-                ++it;
-                continue;
-            }
-            blocks.insert(blocks.end(), it->second.blocks.begin(), it->second.blocks.end());
-            it = g_captures.erase(it);
-        }
+        blocks = captured_blocks(st);
     }
     hipGraph_t g = nullptr;
     hipError_t err = hipStreamEndCapture(st, &g);

@@ -186,6 +186,34 @@ def test_a_callers_own_capture(kt, oracle_lib, kind, sizes):
 
 
 @pytest.mark.parametrize("kind,sizes,larger", KINDS, ids=IDS)
+def test_a_capture_the_caller_ends(kt, oracle_lib, kind, sizes, larger):
+    """Begun with kt_graph_begin and ended with HIP itself: the library does not see this
+    graph's end, so its scratch stays allocated, also after the stream's next graph is gone."""
+    from kotensor_amd import _lib
+    banner("recorded-scratch-callers-end", kind.__name__)
+    call, other = kind(kt, oracle_lib, *sizes, 6), kind(kt, oracle_lib, *larger, 7)
+    want, want_other = call.eager(), other.eager()
+    hip, stream = _hip(), kt.Stream.create()
+    graph, exe = ctypes.c_void_p(), ctypes.c_void_p()
+    _lib.call("kt_graph_begin", stream.handle)
+    try:
+        call.run(stream)
+    finally:
+        assert hip.hipStreamEndCapture(ctypes.c_void_p(stream.handle), ctypes.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, ctypes.c_size_t(0)) == 0
+    assert hip.hipGraphDestroy(graph) == 0
+    with _recorded(other, stream) as later:
+        assert same_bits(_replay(other, later, stream), want_other)
+        assert same_bits(_replay(call, exe, stream), want)
+    kt.release_scratch()
+    for _ in range(2):
+        assert same_bits(_replay(call, exe, stream), want)
+        assert same_bits(other.eager(), want_other)
+    assert hip.hipGraphExecDestroy(exe) == 0
+    stream.destroy()
+
+
+@pytest.mark.parametrize("kind,sizes,larger", KINDS, ids=IDS)
 def test_two_threads_give_the_same_bits(kt, oracle_lib, kind, sizes, larger):
     """Two threads call on the null stream at once: each result has the bits it has alone."""
     import threading
