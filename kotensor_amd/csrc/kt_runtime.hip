@@ -177,9 +177,7 @@ void free_blocks(const std::vector<void*>& blocks) {
     for (void* b : blocks)
         if (hipFree(b) != hipSuccess) (void)hipGetLastError();
 }
-}  // namespace
 
-namespace {
 // `bytes` of the device's pool, in stream order; *out is null if there is no memory left.
 // With g_ws_mutex held.
 int32_t pool_alloc(int device, hipStream_t stream, size_t bytes, void** out) {
@@ -209,10 +207,9 @@ void pool_trim() {
     std::lock_guard<std::mutex> lock(g_ws_mutex);
     if (g_pools[device]) (void)hipMemPoolTrimTo(g_pools[device], 0);
 }
-}  // namespace
 
 // Takes the blocks of the calls recorded since kt_graph_begin on `origin`. With g_ws_mutex held.
-static std::vector<void*> captured_blocks(hipStream_t origin) {
+std::vector<void*> captured_blocks(hipStream_t origin) {
     std::vector<void*> blocks;
     for (auto it = g_captures.begin(); it != g_captures.end();) {
         if (it->second.origin != origin) {
@@ -224,6 +221,7 @@ static std::vector<void*> captured_blocks(hipStream_t origin) {
     }
     return blocks;
 }
+}  // namespace
 
 int32_t CallScratch::take(CallArea kind, hipStream_t stream, size_t bytes) {
     if (t_fixed) {
